@@ -328,9 +328,13 @@ int dense_splits(int chunks, int ztiles, int nks, int cus) {
   return s;
 }
 
-// Large-M path (marlin_dense_prefill_kernel): N a multiple of its 512-column tile, K of
-// 128 (whole scale groups, an even number of 64-deep k-steps) and 32-bit operand
-// offsets, from MARLIN_HIP_DENSE_PREFILL_MIN_M rows (default 65).
+// Large-M path (marlin_dense_prefill_kernel): K a multiple of 128 (whole scale groups, an
+// even number of 64-deep k-steps), N of its 512-column tile, or of half of it (the last
+// tile is then half empty) where that beats the decode-shaped kernel: from 4096 columns,
+// and above 512 rows (us per call, one box: 4096x11008 at M = 65 / 200 / 777 50.8 / 104 /
+// 309 -> 38.2 / 48.4 / 92.7; 4096x2816 at M = 777 / 2000 107 / 208 -> 51.5 / 83.4, but at
+// M = 300 37.4 against 43.3).  32-bit operand offsets; from
+// MARLIN_HIP_DENSE_PREFILL_MIN_M rows (default 65).
 bool dense_prefill_fits(int M, int N, int K) {
   static const int forced_min_m = [] {
     const char* e = getenv("MARLIN_HIP_DENSE_PREFILL_MIN_M");
@@ -338,7 +342,8 @@ bool dense_prefill_fits(int M, int N, int K) {
     return x >= 1 ? x : 0;
   }();
   const int min_m = forced_min_m ? forced_min_m : 65;
-  return M >= min_m && N % kDpTileCols == 0 && K % 128 == 0 && (long long)M * K < (1LL << 31) - 2048 &&
+  const bool cols = N % kDpTileCols == 0 || (N % (kDpTileCols / 2) == 0 && (N >= 4096 || M > 512));
+  return M >= min_m && cols && K % 128 == 0 && (long long)M * K < (1LL << 31) - 2048 &&
          (long long)K * N < (1LL << 33);
 }
 
@@ -381,7 +386,7 @@ int run_dense_prefill(const void* A, const void* B, void* C, const void* s, int 
   p.M = M;
   p.N = N;
   p.K = K;
-  const int tiles = (N / kDpTileCols) * ((M + kDpRows - 1) / kDpRows);
+  const int tiles = ((N + kDpTileCols - 1) / kDpTileCols) * ((M + kDpRows - 1) / kDpRows);
   p.splits = dense_prefill_splits(tiles, K / 64, sms);
   if (p.splits > 1) {
     const int err = get_scratch(dev, stream, (size_t)tiles * p.splits * kDpSplitBytes, &p.counters, &p.partial);

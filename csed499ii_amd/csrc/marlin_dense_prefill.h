@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kDpThreads, 1) void marlin_dense_prefill_kernel(Den
   const int nks = K >> 6;  // even: the host requires K % 128 == 0
 
   // ---- split-K: block b = z * T + tile; split z covers an even range of k-steps ----
-  const int ntn = N / (64 * CT), ntm = (M + MT - 1) / MT;
+  const int ntn = (N + 64 * CT - 1) / (64 * CT), ntm = (M + MT - 1) / MT;
   const int T = ntn * ntm;
   const int S = a.splits;
   int z = 0, tile = blockIdx.x, ks0 = 0, ks1 = nks;
@@ -142,7 +142,10 @@ __global__ __launch_bounds__(kDpThreads, 1) void marlin_dense_prefill_kernel(Den
   const int tn = t / ntm, tm = t - tn * ntm;
   const int c0 = tn * CT;
   const int m0 = tm * MT;
-  const int cw = c0 + w;
+  // chunk of this wave; N is a multiple of 256 columns: in a ragged last tile the waves
+  // past the last chunk compute that one again and store nothing
+  const bool live = c0 + w < N / 64;
+  const int cw = live ? c0 + w : N / 64 - 1;
 
   // ---- DMA sources: per-lane byte offsets from per-k-step bases ----
   // activations: instruction u of wave w fills pieces 64 (2w + u) + lane of the step's
@@ -385,7 +388,7 @@ __global__ __launch_bounds__(kDpThreads, 1) void marlin_dense_prefill_kernel(Den
     float* const pmine = a.partial + ((size_t)tile * S + z) * 65536 + (size_t)w * 8192 + 4 * lane;
 #pragma unroll
     for (int rg = 0; rg < 4; rg++) {
-      if (m0 + 32 * rg >= M) break;  // 32-row blocks past M are never read back (uniform)
+      if (!live || m0 + 32 * rg >= M) break;  // 32-row blocks past M are never read back (uniform)
 #pragma unroll
       for (int hf = 0; hf < 2; hf++)
 #pragma unroll
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(kDpThreads, 1) void marlin_dense_prefill_kernel(Den
   // splits per batch of loads (16 loads in flight per lane). ----
 #pragma unroll
   for (int rg = 0; rg < 4; rg++) {
-    if (m0 + 32 * rg >= M) break;  // uniform: no rows of this block are stored
+    if (!live || m0 + 32 * rg >= M) break;  // uniform: no rows of this block are stored
     float4_t v[2][4];
     if (S == 1) {
 #pragma unroll

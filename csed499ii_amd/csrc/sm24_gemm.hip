@@ -501,7 +501,7 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
   const int max_s = nosplit ? 1 : (nks / 8 > 0 ? nks / 8 : 1);  // at least eight k-steps per split
   if (cus < 1) cus = 1;
   const double exchange_bytes_per_us = 5.0e6;
-  PrefillPlan best{128, 1, (N / kPreTileCols) * ((M + 127) / 128), kPreChunks};
+  PrefillPlan best{128, 1, ((N + kPreTileCols - 1) / kPreTileCols) * ((M + 127) / 128), kPreChunks};
   double best_cost = 1e30;
   // Candidates: 512-column tiles of 128 or 64 rows (the narrow tile, 256 columns x
   // 128 rows of 4 waves, only when forced).  A k-step of a 64-row or narrow tile is
@@ -515,7 +515,7 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
     if ((c.chunks == kPreNarrowChunks) != (forced_chunks == kPreNarrowChunks)) continue;
     if (forced_rows && c.rows != forced_rows) continue;
     if (forced_chunks && c.chunks != forced_chunks) continue;
-    const int tiles = (N / (64 * c.chunks)) * ((M + c.rows - 1) / c.rows);
+    const int tiles = ((N + 64 * c.chunks - 1) / (64 * c.chunks)) * ((M + c.rows - 1) / c.rows);
     if (forced && !nosplit) return PrefillPlan{c.rows, forced < max_s ? forced : max_s, tiles, c.chunks};
     for (int s = 1; s <= 8 && s <= max_s; s++) {
       const long long wgs = (long long)tiles * s, full = wgs / cus, tail = wgs - full * cus;
@@ -543,7 +543,7 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
 
 // A split plan needs one arrival counter per tile (at most 64-row tiles: the most).
 bool prefill_counters_exceed(int N, int M) {
-  return (size_t)(N / kPreTileCols) * ((M + 63) / 64) * sizeof(uint32_t) > kCounterBytes;
+  return (size_t)((N + kPreTileCols - 1) / kPreTileCols) * ((M + 63) / 64) * sizeof(uint32_t) > kCounterBytes;
 }
 
 struct Plan {
@@ -814,8 +814,12 @@ hipError_t launch_decode(const GemmArgs& a, DecodeShape d, int vf, int mf, bool 
   return launch_decode_t<16, false>(a, d, vf, mf, stream);
 }
 
-// Large-M path (sm24_prefill_kernel): 4-bit values and metadata, N a multiple of its
-// 512-column tile and K of its 64-deep k-step, from a batch threshold measured on
+// Large-M path (sm24_prefill_kernel): 4-bit values and metadata, K a multiple of two of
+// its 64-deep k-steps, N of its 512-column tile or, from 1024 columns, of half of it (the
+// last tile is then half empty; against the multi-block kernel, us per call, one box:
+// 4096x11008 at M = 100 / 777 / 2000 65.6 / 300 / 709 -> 23.6 / 54 / 119, 4096x1280 at
+// M = 160 / 777 32.3 / 51.7 -> 21.3 / 24.3; 768 columns keep the multi-block kernel, as
+// callers that query the plan expect), from a batch threshold measured on
 // MI355X against decode launches of <= 32 rows (Llama-2-7B and -70B shapes, M in
 // 48..192, the planner's 64- or 128-row tiles): from M = 33 for the widest N (7B
 // gate_up 4096x22016 at M = 48 / 64: 23.5 / 23.3 against 28.1 / 34.0 us) and for long
@@ -823,15 +827,18 @@ hipError_t launch_decode(const GemmArgs& a, DecodeShape d, int vf, int mf, bool 
 // M = 65 for N >= 4096 (M = 80 / 96: 7B qkv 23.0 / 22.8 against 28.4 / 31.7 us, 7B down
 // 28.2 / 28.5 against 30.3 / 32.8, 70B o 27.9 / 27.5 against 36.1 / 39.7; at M = 48 /
 // 64 the decode launches win for 7B o, down and qkv: 7B o 13.6 / 15.0 against 19.6 /
-// 20.0 us); M >= 160 for narrower N.  MARLIN_HIP_PREFILL_MIN_M (>= 1) replaces the
+// 20.0 us); above the decode launches' 96 rows for narrower N (against the multi-block
+// kernel: 4096x768 at M = 160 43.3 -> 20.6 us, 4096x2816 31.0 -> 20.9, 8192x768 47.1 ->
+// 24.4).  MARLIN_HIP_PREFILL_MIN_M (>= 1) replaces the
 // threshold.
 int prefill_min_m(int N, int K) {
   // the widest N at long K already from 17 rows (70B gate_up 8192x57344 at M = 24 /
   // 32: 49.5 / 50.3 against 58.8 / 67.3 us; at M = 16 49.5 against 49.0)
   if (N >= 16384 && K >= 8192) return 17;
   if (N >= 16384 || (N >= 10240 && K >= 8192)) return kDecodeMaxM + 1;
-  return N >= 4096 ? 65 : 160;
+  return N >= 4096 ? 65 : kDecodeChunkMaxM + 1;
 }
+bool prefill_n(int N) { return N % kPreTileCols == 0 || (N % (kPreTileCols / 2) == 0 && N >= 2 * kPreTileCols); }
 bool prefill_fits(int M, int N, int K, int vf, int mf) {
   static const int forced_min_m = [] {
     const char* e = getenv("MARLIN_HIP_PREFILL_MIN_M");
@@ -839,7 +846,7 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
     return x >= 1 ? x : 0;
   }();
   const int min_m = forced_min_m ? forced_min_m : prefill_min_m(N, K);
-  return vf == VAL4 && mf == META4 && M >= min_m && N % kPreTileCols == 0 && K % 128 == 0 &&
+  return vf == VAL4 && mf == META4 && M >= min_m && prefill_n(N) && K % 128 == 0 &&
          (long long)M * K < (1LL << 31) - 2048 && (long long)K * N < (1LL << 34);
 }
 

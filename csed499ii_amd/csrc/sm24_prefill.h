@@ -132,7 +132,7 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
 
   // ---- split-K: block b = z * T + tile; split z covers the k-steps [ks0, ks1), an even
   // number (>= 8: the host keeps splits <= nks / 8) ----
-  const int ntn = N / (64 * CT), ntm = (M + MT - 1) / MT;
+  const int ntn = (N + 64 * CT - 1) / (64 * CT), ntm = (M + MT - 1) / MT;
   const int T = ntn * ntm;
   const int S = a.splits;
   const int z = blockIdx.x / T;
@@ -159,7 +159,10 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
   }
   const int c0 = tn * CT;         // first chunk of the tile
   const int m0 = tm * MT;         // first batch row
-  const int cw = c0 + w;          // chunk of this wave
+  // chunk of this wave.  N is a multiple of 256 columns: in a ragged last 512-column
+  // tile the waves past the last chunk compute that one again and store nothing.
+  const bool live = c0 + w < N / 64;
+  const int cw = live ? c0 + w : N / 64 - 1;
 
   // ---- DMA sources: per-lane byte offsets from per-k-step bases ----
   // activations: instruction u of wave w fills pieces 64(ADMA w + u) + lane of the
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
     float* const pmine = a.partial + ((size_t)tile * S + z) * PSTRIDE + (size_t)w * (2048 * RG) + 4 * lane;
 #pragma unroll
     for (int rg = 0; rg < RG; rg++) {
-      if (m0 + 32 * rg >= M) break;  // 32-row blocks past M are never read back (uniform)
+      if (!live || m0 + 32 * rg >= M) break;  // 32-row blocks past M are never read back (uniform)
 #pragma unroll
       for (int hf = 0; hf < 2; hf++)
 #pragma unroll
@@ -452,7 +455,7 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
   // uncached reads are latency-bound, so each batch keeps 16 loads in flight. ----
 #pragma unroll
   for (int rg = 0; rg < RG; rg++) {
-    if (m0 + 32 * rg >= M) break;  // uniform: no rows of this block are stored
+    if (!live || m0 + 32 * rg >= M) break;  // uniform: no rows of this block are stored
     float4_t v[2][4];
     if (S == 1) {
 #pragma unroll

@@ -167,6 +167,24 @@ def test_dense_large_m_against_oracle(M, N, K, g):
     assert torch.equal(_run(A, wt), C), "repeated dense large-M calls differ"
 
 
+@pytest.mark.parametrize("M,N,K,g", [(65, 4352, 128, 128), (130, 4352, 2048, -1), (520, 768, 4096, 128),
+                                     (513, 256, 256, -1)])
+def test_dense_large_m_ragged_columns(M, N, K, g):
+    """N a multiple of 256 but not of the 512-column tile (the last tile's upper four
+    waves store nothing): all columns against the oracle, nothing past C's end, and
+    repeated calls bit-identical (split and unsplit along K)."""
+    wt = _dense_weight(K, N, g, M + N + K)
+    A = synth.make_activation(M, K, M + 13, device=DEV)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C = buf[:M * N].view(M, N)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    marlin.mul(A, wt["B"], C, wt["s"], ws)
+    torch.cuda.synchronize()
+    assert_close(C.cpu().numpy(), _oracle(A, wt), f"dense ragged M={M} N={N} K={K} g={g}")
+    assert bool((buf[M * N:] == 7.0).all()), "wrote past C"
+    assert torch.equal(_run(A, wt), C), "repeated calls differ"
+
+
 @pytest.mark.parametrize("M", [512, 2048])
 @pytest.mark.parametrize("K,N", [(8192, 10240), (8192, 57344), (28672, 8192)])
 def test_dense_large_m_llama70b_slices(K, N, M):

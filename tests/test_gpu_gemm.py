@@ -194,6 +194,25 @@ def test_prefill_split_k(M, N, K, g):
         assert torch.equal(_run(wt, A), C), "repeated split-K calls differ"
 
 
+@pytest.mark.parametrize("M,N,K,g", [(97, 1280, 256, 128), (200, 1280, 128, -1), (257, 1792, 8192, 128),
+                                     (65, 4352, 1024, -1), (1100, 2816, 640, 128), (640, 9984, 256, 128)])
+def test_prefill_ragged_columns(M, N, K, g):
+    """Large-M kernel on N a multiple of 256 but not of its 512-column tile: the last
+    tile's upper four waves repeat the last chunk and store nothing (64- and 128-row
+    tiles, narrow tiles, unsplit and split along K); every column against the oracle,
+    nothing past C's end, and repeated calls bit-identical."""
+    assert marlin.plan_2_4(M, K, N, g)["kernel"] == "large_m"
+    wt, A = _problem(M, N, K, g, 5300 + M + N)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C = buf[:M * N].view(M, N)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    marlin.mul_2_4(A, wt["B"], wt["meta"], C, wt["s"], ws)
+    torch.cuda.synchronize()
+    _check(wt, A, C, f"ragged M={M} N={N} K={K} g={g}")
+    assert bool((buf[M * N:] == 7.0).all()), "wrote past C"
+    assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
 @pytest.mark.parametrize("M", [512])
 def test_prefill_shape_slices(M):
     wt, A = _problem(M, 8192, 8192, 128, 31)
