@@ -211,7 +211,7 @@ constexpr int kDecodeChunkMaxM = 96;  // largest batch run as several decode lau
 constexpr int kPreTileCols = 512;
 constexpr int kPreThreads = 512;  // one wave per 64-column chunk of the tile
 constexpr int kPreChunks = 8;        // 64-column chunks per tile = waves per workgroup
-constexpr int kPreNarrowChunks = 4;  // the narrow tile: 256 columns (128 rows), 4 waves
+constexpr int kPreNarrowChunks = 4;  // 256-column tiles: the narrow tile (128 rows, 4 waves) and the two-group tiles
 // fp32 partial of one tile of `rows` (128 or 64) batch rows and `chunks` 64-column chunks
 constexpr size_t pre_split_bytes(int rows, int chunks = 8) { return (size_t)64 * chunks * rows * sizeof(float); }
 hipError_t launch_prefill(const GemmArgs& a, int rows, int chunks, bool grouped, hipStream_t stream);

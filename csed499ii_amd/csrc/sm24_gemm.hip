@@ -474,11 +474,20 @@ __global__ __launch_bounds__(256) void w3_to_w4_kernel(const uint32_t* __restric
 // Llama-2-70B qkv and o at M = 512 and 1024, one box: 0.61-0.71, the higher at low
 // occupancy).
 constexpr double kPreNarrowStep = 0.66;
+// The two-group tiles (sm24_prefill.h) replace the 64-row 512-column ones up to this
+// batch (three 64-row or two 96-row tiles).  Forced plans over Llama-2-7B and -70B shapes
+// at M in {64, 96, 131, 160, 192}, one box (us per call, 64-row 512-column tiles -> this
+// planner's choice): M = 131 7B qkv 26.0 -> 21.4, o 20.3 -> 15.6, gate_up 34.7 -> 31.2,
+// down 30.6 -> 23.2, 70B o 31.9 -> 27.2, qkv 35.9 -> 30.2; 7B gate_up at M = 96 31.4 ->
+// 24.9; no call of the sweep was faster on the 512-column tiles.  The planner's choices
+// sum to 629.9 us against 626.6 for the best forced plan of each call.
+constexpr int kPreGroupMaxM = 192;
 struct PrefillPlan {
-  int rows;    // batch rows per tile: 128 or 64
+  int rows;    // batch rows per tile: 128, 64 or (two k-groups) 96
   int splits;  // K splits
   int tiles;   // tiles (workgroups per split)
-  int chunks;  // 64-column chunks per tile (= waves): 8, or 4 for the narrow 128-row tile
+  int chunks;  // 64-column chunks per tile: 8, or 4 for the narrow 128-row tile and the two-group tiles
+  int waves() const { return chunks == kPreNarrowChunks && rows < 128 ? 2 * chunks : chunks; }
 };
 // k-step time (us) of a 128-row tile with a fraction x of the CUs busy (measured).
 double prefill_step_us(double x) {
@@ -495,7 +504,7 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
     const int x = e ? atoi(e) : 0;
     return x >= 1 && x <= 16 ? x : 0;
   }();
-  static const int forced_rows = env_choice("MARLIN_HIP_PREFILL_ROWS", {64, 128}, 0);
+  static const int forced_rows = env_choice("MARLIN_HIP_PREFILL_ROWS", {64, 96, 128}, 0);
   static const int forced_chunks = env_choice("MARLIN_HIP_PREFILL_CHUNKS", {kPreNarrowChunks, kPreChunks}, 0);
   const int nks = K / 64;
   const int max_s = nosplit ? 1 : (nks / 8 > 0 ? nks / 8 : 1);  // at least eight k-steps per split
@@ -503,24 +512,35 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
   const double exchange_bytes_per_us = 5.0e6;
   PrefillPlan best{128, 1, ((N + kPreTileCols - 1) / kPreTileCols) * ((M + 127) / 128), kPreChunks};
   double best_cost = 1e30;
-  // Candidates: 512-column tiles of 128 or 64 rows (the narrow tile, 256 columns x
-  // 128 rows of 4 waves, only when forced).  A k-step of a 64-row or narrow tile is
-  // a fraction `hscale` of a 512x128 one at the same occupancy.
+  // Candidates: 512-column tiles of 128 or 64 rows, the two-group tiles of 256 columns
+  // (the narrow tile, 256 columns x 128 rows of 4 waves, only when forced).  A k-step of
+  // another tile is a fraction `hscale` of a 512x128 one at the same occupancy.
   struct Cand {
-    int rows, chunks;
+    int rows, chunks, groups;
     double hscale;
   };
-  const Cand cands[] = {{128, kPreChunks, 1.0}, {64, kPreChunks, 0.63}, {128, kPreNarrowChunks, kPreNarrowStep}};
+  const Cand cands[] = {{128, kPreChunks, 1, 1.0},
+                        {64, kPreChunks, 1, 0.63},
+                        {128, kPreNarrowChunks, 1, kPreNarrowStep},
+                        {64, kPreNarrowChunks, 2, 0.69},
+                        {96, kPreNarrowChunks, 2, 1.15}};
+  // Up to kPreGroupMaxM rows the two-group tiles replace the 64-row 512-column ones.
+  const bool groups = (M <= kPreGroupMaxM || forced_rows) && nks >= 16 && forced_chunks != kPreChunks;
   for (const Cand& c : cands) {
-    if ((c.chunks == kPreNarrowChunks) != (forced_chunks == kPreNarrowChunks)) continue;
+    if (c.groups == 1 && (c.chunks == kPreNarrowChunks) != (forced_chunks == kPreNarrowChunks)) continue;
+    if (c.groups > 1 && !groups) continue;
+    if (c.rows == 64 && c.groups == 1 && groups && !forced_rows) continue;
     if (forced_rows && c.rows != forced_rows) continue;
     if (forced_chunks && c.chunks != forced_chunks) continue;
     const int tiles = ((N + 64 * c.chunks - 1) / (64 * c.chunks)) * ((M + c.rows - 1) / c.rows);
-    if (forced && !nosplit) return PrefillPlan{c.rows, forced < max_s ? forced : max_s, tiles, c.chunks};
-    for (int s = 1; s <= 8 && s <= max_s; s++) {
+    const int cmax_s = max_s / c.groups > 0 ? max_s / c.groups : 1;
+    if (forced && !nosplit) return PrefillPlan{c.rows, forced < cmax_s ? forced : cmax_s, tiles, c.chunks};
+    for (int s = 1; s <= 8 && s <= cmax_s; s++) {
+      if (s > 1 && (size_t)tiles * sizeof(uint32_t) > kCounterBytes) break;  // one arrival counter per tile
       const long long wgs = (long long)tiles * s, full = wgs / cus, tail = wgs - full * cus;
       double cost = ((double)full * prefill_step_us(1.0) + (tail ? prefill_step_us((double)tail / cus) : 0.0)) *
-                    c.hscale * nks / s;
+                    c.hscale * nks / (s * c.groups);
+      if (c.groups > 1) cost += 1.0;  // the groups' accumulators, exchanged through LDS
       if (s > 1) cost += 2.0 * tiles * s * (double)pre_split_bytes(c.rows, c.chunks) / exchange_bytes_per_us;
       if (cost < 0.98 * best_cost) {
         best_cost = cost;
@@ -909,7 +929,7 @@ void describe(int M, int N, int K, int sms, bool noalloc, int out[5]) {
   } else if (kernel == KERNEL_PREFILL) {
     const PrefillPlan pp = prefill_plan(M, N, K, sms, noalloc || prefill_counters_exceed(N, M));
     out[1] = pp.tiles * pp.splits;
-    out[2] = 64 * pp.chunks;
+    out[2] = 64 * pp.waves();
     out[3] = pp.splits;
     out[4] = 1;
   } else {

@@ -10,6 +10,12 @@
 // SIMD, one workgroup per CU by its 92 KiB of LDS), the same per-wave work as the
 // 512-column tile; it replaces 64-row tiles where it comes to the same number of
 // workgroups, so that each dequantized weight fragment still feeds four B fragments.
+// The two-group tile (CT = 4, KG = 2; 256 columns x 64 or 96 rows, 8 waves) runs two
+// k-groups of 4 waves on the two halves of the workgroup's k-steps, each with its own
+// ring, and adds their accumulators in LDS: at 65 to a few hundred rows a 512-column
+// 64-row tile must split K across workgroups to fill the chip, and its exchange through
+// uncached memory costs as much as its MFMAs; twice the tiles at half the k-steps need
+// half the splits or none.
 //
 // Why two waves per SIMD.  Measured on MI355X (random operands): a 32x32x32 smfmac
 // takes ~35 cycles, and the VALU can issue ~4 instructions of 4 cycles beside it.
@@ -68,7 +74,9 @@ struct PreLds {
   static constexpr int bytes = wgt_off + kPreRing * wgt_b;
 };
 static_assert(kPreWgtW % 256 == 0, "wave blocks keep the bank pattern");
-static_assert(PreLds<4>::bytes <= 160 * 1024 && PreLds<4, kPreNarrowChunks>::bytes <= 96 * 1024, "LDS");
+static_assert(PreLds<4>::bytes <= 160 * 1024 && PreLds<4, kPreNarrowChunks>::bytes <= 96 * 1024 &&
+                  2 * PreLds<3, kPreNarrowChunks>::bytes <= 160 * 1024,
+              "LDS");
 
 // v_smfmac_f32_32x32x32_f16 with the accumulator in AGPRs; ABID selects the index
 // halfword.  Written as inline assembly because, for the intrinsic, the compiler
@@ -98,20 +106,22 @@ __device__ __forceinline__ void pre_step_barrier() {
 
 // First dequantization slice of MFMA region r of a k-step with nr regions: the 14
 // slices of the next step's two k-blocks run in regions 2..nr-1, one per region with
-// 16 regions, with 8 three or two per region (k-block 0 in regions 2-4, 1 in 5-7).
+// 16 regions, with 8 three or two per region (k-block 0 in regions 2-4, 1 in 5-7), with
+// 12 one or two.
 constexpr int pre_slice0(int nr, int r) {
-  return r <= 2 ? 0 : nr == 16 ? r - 2 : r == 3 ? 3 : r == 4 ? 5 : r == 5 ? 7 : r == 6 ? 10 : r == 7 ? 12 : 14;
+  return r <= 2 ? 0 : nr == 16 ? r - 2 : nr == 12 ? (r - 2) * 14 / 10 : r == 3 ? 3 : r == 4 ? 5 : r == 5 ? 7 : r == 6 ? 10 : r == 7 ? 12 : 14;
 }
-static_assert(pre_slice0(16, 16) == 14 && pre_slice0(8, 8) == 14, "every slice once");
+static_assert(pre_slice0(16, 16) == 14 && pre_slice0(12, 12) == 14 && pre_slice0(8, 8) == 14, "every slice once");
 
 // RG: 32-row B fragments per wave, i.e. a tile of 32 RG batch rows.  RG = 4 is the
 // tile described above; RG = 2 (64 rows) doubles the tiles of a call for batches whose
 // 128-row tiles leave CUs idle, at twice the dequantization per MFMA (each weight
 // fragment feeds two B fragments instead of four: ~6.5 VALU per MFMA).
-template <bool GROUPED, int RG, int CT>
-__global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
-  static_assert(RG == 4 || RG == 2, "128- or 64-row tiles");
-  static_assert(CT == kPreChunks || (CT == kPreNarrowChunks && RG == 4), "512- or (128-row) 256-column tiles");
+// KG: k-groups of CT waves, each on its share of the workgroup's k-steps.
+template <bool GROUPED, int RG, int CT, int KG = 1>
+__global__ __launch_bounds__(64 * CT * KG, 1) void sm24_prefill_kernel(GemmArgs a) {
+  static_assert(KG == 1 ? RG == 4 || (RG == 2 && CT == kPreChunks) : KG == 2 && RG <= 3 && CT == kPreNarrowChunks,
+                "128-row tiles, 64-row tiles of 512 columns, or two k-groups of 256 columns");
   constexpr int MT = 32 * RG;
   constexpr int NF = 2 * RG;               // B fragments per k-step (two k-blocks)
   constexpr int NR = 2 * NF;               // MFMA regions per k-step
@@ -120,13 +130,15 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
   constexpr int kPreActB = PreLds<RG, CT>::act_b, kPreWgtOff = PreLds<RG, CT>::wgt_off;
   constexpr int kPreWgtB = PreLds<RG, CT>::wgt_b;
   constexpr int PSTRIDE = 2048 * CT * RG;  // floats of one (tile, split) partial
-  __shared__ __attribute__((aligned(16))) uint8_t lds[PreLds<RG, CT>::bytes];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_all[KG * PreLds<RG, CT>::bytes];
   typedef __attribute__((address_space(3))) uint8_t lds_u8;
-  const uint32_t lbase = (uint32_t)(size_t)(lds_u8*)lds;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // chunk of this wave
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = KG == 1 ? wv : wv % CT, kg = KG == 1 ? 0 : wv / CT;  // chunk and k-group of this wave
+  uint8_t* const lds = lds_all + kg * PreLds<RG, CT>::bytes;         // its group's ring
+  const uint32_t lbase = (uint32_t)(size_t)(lds_u8*)lds_all + kg * PreLds<RG, CT>::bytes;
   const int M = a.M, N = a.N, K = a.K;
   const int nks = K >> 6;  // even: the host requires K % 128 == 0
 
@@ -136,8 +148,9 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
   const int T = ntn * ntm;
   const int S = a.splits;
   const int z = blockIdx.x / T;
-  const int ks0 = 2 * (int)(((long long)(nks >> 1) * z) / S);
-  const int ks1 = 2 * (int)(((long long)(nks >> 1) * (z + 1)) / S);
+  const int kz = z * KG + kg;  // k-group's share of all splits' k-steps
+  const int ks0 = 2 * (int)(((long long)(nks >> 1) * kz) / (S * KG));
+  const int ks1 = 2 * (int)(((long long)(nks >> 1) * (kz + 1)) / (S * KG));
 
   // ---- tile order: each XCD (block b on XCD b % 8) works through a contiguous range
   // of tiles, in supertiles of GN column tiles x GM row tiles (rows fastest), so that
@@ -212,10 +225,11 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
         dma16x1(la, act_v[0], gA1 + 128 * sc);
       } else {
 #pragma unroll
-        for (int u = 0; u < ADMA; u += 2) {
+        for (int u = 0; u + 1 < ADMA; u += 2) {
           const uint32_t pair[2] = {act_v[u], act_v[u + 1]};
           dma16x2(la + 1024 * u, pair, gA1 + 128 * sc);
         }
+        if constexpr (ADMA % 2) dma16x1(la + 1024 * (ADMA - 1), act_v[ADMA - 1], gA1 + 128 * sc);
       }
     } else {
       const uint32_t l = lbase + kPreWgtOff + q * kPreWgtB + kPreWgtW * w;
@@ -254,7 +268,8 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
 
   half8_t av[2][2][2];  // [parity][kb][hf] dequantized weight fragments
   uint32_t ix[2][2];    // [parity][kb] index halfwords (hf = abid)
-  half16_t bv[4];       // B fragments, ring by fragment number kb*RG + rg
+  constexpr int BR = NF % 4 == 0 ? 4 : 3;  // ring of B fragments: divides a k-step's
+  half16_t bv[BR];      // B fragments, ring by fragment number kb*RG + rg
   f32x16 acc[RG][2];    // [rg][hf]
 #pragma unroll
   for (int rg = 0; rg < RG; rg++)
@@ -357,7 +372,7 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
   //   barrier: this wave's DMAs of step s+1 have landed, every wave has finished step
   //   s-1 (its reads of slot Q+3);
   //   NR = 4 RG regions r = (kb, rg, hf), each one MFMA plus a share of: DMA group
-  //   r >> 1 of step s+3 (r = 1, 3); at hf = 0 the read of B fragment f+3 (f = RG kb +
+  //   r >> 1 of step s+3 (r = 1, 3); at hf = 0 the read of B fragment f+BR-1 (f = RG kb +
   //   rg; from step s+1 past NF-1; its ring slot held fragment f-1, used up by then);
   //   at r < 2 the raw words and metadata of step s+1, k-block r, and at r = 2 its
   //   scales; at r >= 2 the slices [pre_slice0(r), pre_slice0(r+1)) of dequantizing
@@ -370,10 +385,10 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const int kb = r / (2 * RG), rg = (r >> 1) % RG, hf = r & 1, f = r >> 1;
-      if (hf) pre_smfmac<1>(acc[rg][hf], av[P][kb][hf], bv[f & 3], ix[P][kb]);
-      else pre_smfmac<0>(acc[rg][hf], av[P][kb][hf], bv[f & 3], ix[P][kb]);
+      if (hf) pre_smfmac<1>(acc[rg][hf], av[P][kb][hf], bv[f % BR], ix[P][kb]);
+      else pre_smfmac<0>(acc[rg][hf], av[P][kb][hf], bv[f % BR], ix[P][kb]);
       __builtin_amdgcn_sched_barrier(0);  // the region's work follows its MFMA
-      if (hf == 0) bv[(f + 3) & 3] = read_b(f + 3 < NF ? Q : QN, (f + 3) % NF);
+      if (hf == 0) bv[(f + BR - 1) % BR] = read_b(f + BR - 1 < NF ? Q : QN, (f + BR - 1) % NF);
       if (r == 1 || r == 3) dma(s + 3, QD, r >> 1);
       if (r < 2) read_raw(QN, r);
       if (r == 2) read_scales(QN);
@@ -399,16 +414,37 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
     for (int sl = 0; sl < 7; sl++) dq_slice(kb, sl, 0);
   bv[0] = read_b(0, 0);
   bv[1] = read_b(0, 1);
-  bv[2] = read_b(0, 2);
+  if constexpr (BR > 3) bv[2] = read_b(0, 2);
   __builtin_amdgcn_sched_barrier(0);
 
-  const int nls = ks1 - ks0;  // k-steps of this split (even)
-  for (int s = 0; s < nls; s += 4) {
-    step(s, IntC<0>{});
-    step(s + 1, IntC<1>{});
-    if (s + 2 < nls) {
-      step(s + 2, IntC<2>{});
-      step(s + 3, IntC<3>{});
+  const int nls = ks1 - ks0;  // k-steps of this split and k-group (even)
+  if constexpr (KG == 1) {
+    for (int s = 0; s < nls; s += 4) {
+      step(s, IntC<0>{});
+      step(s + 1, IntC<1>{});
+      if (s + 2 < nls) {
+        step(s + 2, IntC<2>{});
+        step(s + 3, IntC<3>{});
+      }
+    }
+  } else {
+    // the groups' shares differ by at most one pair of steps: the shorter one meets the
+    // longer one's last two barriers without work
+    const int e0 = 2 * (int)(((long long)(nks >> 1) * (z * KG)) / (S * KG));
+    const int e1 = 2 * (int)(((long long)(nks >> 1) * (z * KG + 1)) / (S * KG));
+    const int e2 = 2 * (int)(((long long)(nks >> 1) * (z * KG + 2)) / (S * KG));
+    const int nmax = e1 - e0 > e2 - e1 ? e1 - e0 : e2 - e1;
+    for (int s = 0; s < nls; s += 4) {
+      step(s, IntC<0>{});
+      step(s + 1, IntC<1>{});
+      if (s + 2 < nls) {
+        step(s + 2, IntC<2>{});
+        step(s + 3, IntC<3>{});
+      }
+    }
+    if (nls < nmax) {
+      pre_step_barrier<NDMA>();
+      pre_step_barrier<NDMA>();
     }
   }
   // DMAs of (clamped) steps past the last may still be landing in LDS
@@ -418,6 +454,37 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
   for (int rg = 0; rg < RG; rg++)
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) asm volatile("" : "+a"(acc[rg][hf]));
+
+  // ---- two k-groups: group rg % 2 takes over 32-row block rg, the other one hands its
+  // accumulators over through LDS (group 0's sum first) ----
+  auto owns = [&](int rg) { return KG == 1 || (rg & 1) == kg; };
+  if constexpr (KG == 2) {
+    __syncthreads();  // the last steps' reads of the rings are done
+    float* const xch = reinterpret_cast<float*>(lds_all) + w * (2048 * RG) + 4 * lane;
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++)
+      if (!owns(rg)) {
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            *reinterpret_cast<float4_t*>(xch + ((rg * 2 + hf) * 4 + i) * 256) = (float4_t){
+                acc[rg][hf][4 * i], acc[rg][hf][4 * i + 1], acc[rg][hf][4 * i + 2], acc[rg][hf][4 * i + 3]};
+      }
+    __syncthreads();
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++)
+      if (owns(rg)) {
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const float4_t o = *reinterpret_cast<const float4_t*>(xch + ((rg * 2 + hf) * 4 + i) * 256);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[rg][hf][4 * i + e] += o[e];
+          }
+      }
+  }
 
   // ---- split-K hand-off: the partial tile goes to uncached scratch in register order
   // ([tile][split][wave][rg][hf][i][lane] float4s, 64 RG KiB per tile and split); the
@@ -431,6 +498,7 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
 #pragma unroll
     for (int rg = 0; rg < RG; rg++) {
       if (!live || m0 + 32 * rg >= M) break;  // 32-row blocks past M are never read back (uniform)
+      if (!owns(rg)) continue;
 #pragma unroll
       for (int hf = 0; hf < 2; hf++)
 #pragma unroll
@@ -456,6 +524,7 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
 #pragma unroll
   for (int rg = 0; rg < RG; rg++) {
     if (!live || m0 + 32 * rg >= M) break;  // uniform: no rows of this block are stored
+    if (!owns(rg)) continue;
     float4_t v[2][4];
     if (S == 1) {
 #pragma unroll
@@ -498,5 +567,8 @@ __global__ __launch_bounds__(64 * CT, 1) void sm24_prefill_kernel(GemmArgs a) {
     }
   }
 }
+
+// The two-group tiles' launcher (sm24_prefill_groups.hip).
+hipError_t launch_prefill_groups(const GemmArgs& a, int rows, bool grouped, dim3 grid, hipStream_t stream);
 
 }  // namespace sm24

@@ -6,6 +6,7 @@ namespace sm24 {
 hipError_t launch_prefill(const GemmArgs& a, int rows, int chunks, bool grouped, hipStream_t stream) {
   const dim3 grid(((a.N + 64 * chunks - 1) / (64 * chunks)) * ((a.M + rows - 1) / rows) * a.splits);
   constexpr int W = kPreChunks, NW = kPreNarrowChunks;
+  if (chunks == NW && rows < 128) return launch_prefill_groups(a, rows, grouped, grid, stream);
   if (chunks == NW) {  // 128-row tiles of 256 columns, 4 waves
     if (grouped) hipLaunchKernelGGL((sm24_prefill_kernel<true, 4, NW>), grid, dim3(64 * NW), 0, stream, a);
     else hipLaunchKernelGGL((sm24_prefill_kernel<false, 4, NW>), grid, dim3(64 * NW), 0, stream, a);

@@ -194,6 +194,26 @@ def test_prefill_split_k(M, N, K, g):
         assert torch.equal(_run(wt, A), C), "repeated split-K calls differ"
 
 
+@pytest.mark.parametrize("M,N,K,g", [(65, 4096, 1024, 128), (97, 1280, 1152, 128), (128, 4352, 1152, -1),
+                                     (129, 4096, 2176, 128), (131, 8192, 1024, -1), (192, 4096, 8192, 128),
+                                     (161, 1024, 11008, 128), (96, 10240, 8192, 128), (192, 22016, 1024, 128)])
+def test_prefill_two_group_tiles(M, N, K, g):
+    """Two k-groups per workgroup (65-192 rows, K from 1024): 64- and 96-row tiles,
+    equal and unequal shares of the k-steps (K = 1152: 4 and 5 pairs), ragged rows,
+    unsplit and split along K; against the oracle, repeated calls bit-identical."""
+    p = marlin.plan_2_4(M, K, N, g)
+    assert p["kernel"] == "large_m" and p["threads"] == 512
+    wt, A = _problem(M, N, K, g, 6100 + M + K)
+    C = _run(wt, A)
+    assert torch.isfinite(C).all()
+    t = to_cpu(wt)
+    for c0 in (0, N // 128, N // 64 - 4):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"M={M} {K}x{N} g={g} slice {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
 @pytest.mark.parametrize("M,N,K,g", [(97, 1280, 256, 128), (200, 1280, 128, -1), (257, 1792, 8192, 128),
                                      (65, 4352, 1024, -1), (1100, 2816, 640, 128), (640, 9984, 256, 128)])
 def test_prefill_ragged_columns(M, N, K, g):

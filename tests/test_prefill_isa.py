@@ -195,6 +195,22 @@ def test_prefill_registers(prefill_asm):
     assert prefill_asm.count("; NumAgprs: 64") == 2
 
 
+def test_prefill_two_group_tiles(tmp_path_factory):
+    """The two-group tiles (256 columns x 64 or 96 rows, two k-groups of 4 waves): the
+    same hazard rules, no scratch, 64 or 96 accumulators in AGPRs, and at most 256
+    registers in all, so that the workgroup's 8 waves are resident."""
+    asm = _compile(ROOT / "csed499ii_amd" / "csrc" / "sm24_prefill_groups.hip", tmp_path_factory)
+    kernels = _kernels(asm)
+    assert len(kernels) == 4
+    for name, body in kernels.items():
+        assert sum(1 for l in body.split("\n") if "v_smfmac" in l) >= (32 if "Li2ELi4ELi2E" in name else 48), name
+        assert hazards(body) == [], name
+    for m in re.finditer(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", asm, re.S):
+        assert int(re.search(r"\.amdhsa_private_segment_fixed_size\s+(\d+)", m.group(2)).group(1)) == 0, m.group(1)
+        assert int(re.search(r"\.amdhsa_next_free_vgpr\s+(\d+)", m.group(2)).group(1)) <= 256, m.group(1)
+    assert sorted(re.findall(r"; NumAgprs: (\d+)", asm)) == ["64", "64", "96", "96"]
+
+
 def test_dense_prefill_mfma_hazards(dense_prefill_asm):
     kernels = _kernels(dense_prefill_asm, "marlin_dense_prefill_kernel")
     assert len(kernels) == 2  # grouped and per-column scales
