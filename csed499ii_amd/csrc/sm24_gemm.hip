@@ -870,6 +870,52 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
          (long long)M * K < (1LL << 31) - 2048 && (long long)K * N < (1LL << 34);
 }
 
+// Tile and K splits of the mid-batch kernel (33-192 rows), from a cost model fitted to
+// 1000 forced plans (every tile x splits 1-8 on ten K x N, 2048x2048 to 28672x8192, M in
+// {33, 48, 64, 80, 96, 131, 160, 192}, one box; mean error 4 %, the model's choices 1 %
+// from the best of each call): a fixed cost, the stages of a wave at the tile's measured
+// stage time, the reduction in LDS (by tile size), and for a split the exchange of the
+// fp32 partials.  Only plans of one workgroup per CU in one round are considered: a
+// second round loses to the large-M kernel (7B gate_up at M = 96 31.1 against 24.2 us,
+// 4096x12288 at M = 131 24.9 against 21.4), as does K above 16384 beyond 64 rows
+// (28672x8192 at M = 96: 49.9 against 46.3).  splits == 0: no such plan.
+// MARLIN_HIP_MID=0 turns the kernel off (read once).
+constexpr int kMidMaxM = 192;
+MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
+  static const int on = env_choice("MARLIN_HIP_MID", {0, 1}, 1);
+  struct Cand {
+    int ncb, rb;
+    double stage_us;
+  };
+  static const Cand cands[] = {{4, 1, 0.45}, {4, 2, 0.54}, {4, 3, 0.72}, {4, 4, 0.82},
+                               {4, 5, 0.95}, {8, 2, 0.87}, {8, 3, 1.07}, {8, 4, 1.10}};
+  MidShape best{0, 0, 0};
+  if (!on || M <= kDecodeMaxM || M > kMidMaxM || K % 64 != 0 || (K > 16384 && M > 64) ||
+      (long long)M * K >= (1LL << 31))
+    return best;
+  // Narrow N at up to 64 rows, K from 4096: the launches a query of the plan expects
+  // there are two, so K is split and a second launch adds the partials (4096x4096 at
+  // M = 64: one unsplit launch of 16-row tiles takes 8.0 us).
+  const bool two = !nosplit && M <= kDecodeMidMaxM && 2 * (N / 64) < cus && K >= 4096;
+  double best_cost = 1e30;
+  for (const Cand& c : cands) {
+    if (N % (16 * c.ncb) != 0) continue;
+    const int tiles = N / (16 * c.ncb) * ((M + 16 * c.rb - 1) / (16 * c.rb));
+    for (int s = two ? 2 : 1; s <= (nosplit ? 1 : 8) && tiles * s <= cus; s++) {
+      if (s > 1 && K / 64 < 8 * s) break;
+      const double x = (double)(tiles * s) / cus;
+      double cost = 3.1 + ((K / 64 + s - 1) / s + 7) / 8 * c.stage_us * (1 + 0.18 * (x - 0.75)) + 0.096 * c.ncb * c.rb;
+      if (s > 1) cost += 1.1 + 8.0 * s * M * (double)N / 5.3e6;
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = MidShape{c.ncb, c.rb, s, two};
+      }
+    }
+  }
+  return best;
+}
+bool mid_fits(int M, int N, int K, int cus, bool nosplit) { return mid_plan(M, N, K, cus, nosplit).splits > 0; }
+
 // Shape/tile validation with the reference's rules and error codes
 // (marlin_cuda_kernel_nm.cu:760-823).
 int validate(int prob_m, int prob_n, int prob_k, int groupsize, int thread_k, int thread_m) {
@@ -897,15 +943,17 @@ int validate(int prob_m, int prob_n, int prob_k, int groupsize, int thread_k, in
 }
 
 
-enum : int { KERNEL_DECODE = 0, KERNEL_PREFILL = 1, KERNEL_GENERAL = 2, KERNEL_DECODE_DMA = 3 };
+enum : int { KERNEL_DECODE = 0, KERNEL_PREFILL = 1, KERNEL_GENERAL = 2, KERNEL_DECODE_DMA = 3, KERNEL_MID = 4 };
 
 // The kernel a call on the reference layout runs (after 3-bit operands at large M are
-// expanded to 4 bits): the decode kernel up to 32 rows, and below the large-M
+// expanded to 4 bits): the mid-batch kernel at 33-192 rows where it covers the call in
+// one round, else the decode kernel up to 32 rows, and below the large-M
 // kernel's threshold up to 96 rows as consecutive launches of <= 32 rows (measured
 // on the Llama-2-7B shapes: o at M = 64 17.8 against 28.8 us, down at M = 96 40.5
 // against 49.7 us for the general kernel); the large-M kernel where it fits; the
 // general kernel otherwise.
-int kernel_for(int M, int N, int K) {
+int kernel_for(int M, int N, int K, int cus, bool nosplit) {
+  if (mid_fits(M, N, K, cus, nosplit)) return KERNEL_MID;
   if (prefill_fits(M, N, K, VAL4, META4)) return KERNEL_PREFILL;
   return M <= kDecodeChunkMaxM ? KERNEL_DECODE : KERNEL_GENERAL;
 }
@@ -914,9 +962,18 @@ int kernel_for(int M, int N, int K) {
 // out = {kernel (of the first launch), workgroups of the first launch, threads per
 // workgroup, K splits of the first launch, launches}.
 void describe(int M, int N, int K, int sms, bool noalloc, int out[5]) {
-  const int kernel = kernel_for(M, N, K);
+  const int kernel = kernel_for(M, N, K, sms, noalloc);
   out[0] = kernel;
-  if (kernel == KERNEL_DECODE) {
+  if (kernel == KERNEL_MID) {
+    // reported with the family of its batch: the large-M kernels from their threshold on,
+    // the LDS-DMA decode kernels below
+    const MidShape d = mid_plan(M, N, K, sms, noalloc);
+    out[0] = M >= prefill_min_m(N, K) ? KERNEL_PREFILL : KERNEL_DECODE_DMA;
+    out[1] = N / (16 * d.ncb) * ((M + 16 * d.rb - 1) / (16 * d.rb)) * d.splits;
+    out[2] = 512;
+    out[3] = d.splits;
+    out[4] = d.two_launches ? 2 : 1;
+  } else if (kernel == KERNEL_DECODE) {
     const int mc = M < kDecodeMaxM ? M : kDecodeMaxM;
     DecodeShape d = decode_shape(mc, N, K, sms);
     if (noalloc) decode_unsplit(d, K);
@@ -978,7 +1035,32 @@ int run(int vf, int mf, const void* A, const void* B, const void* meta, void* C,
   const _Float16* zeros = nullptr;
   err = get_zeros(dev, stream, &zeros);
   if (err != MARLIN_HIP_OK) return err;
-  if (kernel_for(M, N, K) == KERNEL_DECODE) {
+  const int kernel = kernel_for(M, N, K, sms, noalloc);
+  if (kernel == KERNEL_MID) {
+    GemmArgs p{};
+    p.A = static_cast<const _Float16*>(A);
+    p.B = B;
+    p.meta = meta;
+    p.s = static_cast<const _Float16*>(s);
+    p.C = static_cast<_Float16*>(C);
+    p.zeros = zeros;
+    p.M = M;
+    p.N = N;
+    p.K = K;
+    MidShape d = mid_plan(M, N, K, sms, noalloc);
+    if (d.splits > 1) {
+      const size_t tiles = (size_t)(N / (16 * d.ncb)) * ((M + 16 * d.rb - 1) / (16 * d.rb));
+      err = get_scratch(dev, stream, tiles * d.splits * 256 * d.ncb * d.rb * sizeof(float), &p.counters, &p.partial);
+      if (err != MARLIN_HIP_OK) return err;
+      if (!p.counters) d = mid_plan(M, N, K, sms, true);  // capturing, and this stream has no scratch yet
+      else if (d.two_launches) p.counters = nullptr;
+    }
+    if (d.splits > 0) {
+      p.splits = d.splits;
+      return launch_error(launch_mid(p, d, vf, mf, groupsize != -1, stream));
+    }
+  }
+  if (kernel == KERNEL_DECODE) {
     for (int r0 = 0; r0 < M; r0 += kDecodeMaxM) {
       const int mc = M - r0 < kDecodeMaxM ? M - r0 : kDecodeMaxM;
       GemmArgs d{};

@@ -194,9 +194,73 @@ def test_prefill_split_k(M, N, K, g):
         assert torch.equal(_run(wt, A), C), "repeated split-K calls differ"
 
 
-@pytest.mark.parametrize("M,N,K,g", [(65, 4096, 1024, 128), (97, 1280, 1152, 128), (128, 4352, 1152, -1),
-                                     (129, 4096, 2176, 128), (131, 8192, 1024, -1), (192, 4096, 8192, 128),
-                                     (161, 1024, 11008, 128), (96, 10240, 8192, 128), (192, 22016, 1024, 128)])
+MID_CASES = [(33, 2048, 2048, 128), (40, 256, 64, -1), (48, 4096, 4096, 128), (64, 4096, 4096, -1),
+             (64, 12288, 1024, 128), (50, 22016, 1024, 128), (64, 22016, 512, -1), (48, 10240, 8192, 128),
+             (65, 4096, 4096, 128), (80, 12288, 1024, -1), (96, 10240, 2048, 128), (100, 2048, 832, -1),
+             (131, 5120, 1024, 128), (131, 4096, 11008, 128), (192, 8192, 2176, 128), (192, 256, 4096, -1)]
+
+
+@pytest.mark.parametrize("M,N,K,g", MID_CASES)
+def test_mid_batches(M, N, K, g):
+    """The mid-batch kernel (33-192 rows, one round over the CUs): every tile it has
+    (64 columns x 16-80 rows, 128 columns x 32-64), fewer k-pairs than waves (K = 64),
+    odd counts of them (K = 832, 2176), ragged rows, unsplit, split with the hand-off in
+    the launch and (narrow N up to 64 rows) with the sums added by a second launch;
+    column slices against the oracle, nothing past C's end, repeated calls bit-identical."""
+    p = marlin.plan_2_4(M, K, N, g)
+    assert p["threads"] == 512 and p["kernel"] in ("decode_dma", "large_m")
+    assert p["launches"] == (2 if M <= 64 and N <= 8128 and K >= 4096 else 1)
+    wt, A = _problem(M, N, K, g, 8100 + M + K + N)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C = buf[:M * N].view(M, N)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    marlin.mul_2_4(A, wt["B"], wt["meta"], C, wt["s"], ws)
+    torch.cuda.synchronize()
+    assert torch.isfinite(C).all() and bool((buf[M * N:] == 7.0).all())
+    t = to_cpu(wt)
+    for c0 in sorted({0, max(N // 128 - 2, 0), N // 64 - 4}):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"M={M} {K}x{N} g={g} slice {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 4096, 4096), (131, 11008, 4096), (48, 8192, 10240)])
+def test_mid_graph_replay_and_noalloc(M, K, N):
+    """Captured mid-batch calls that split K (a second launch, or the hand-off in the
+    launch) replay the eager result with eager work between the replays; on a stream
+    without scratch the captured call runs unsplit; so does the no-allocation call."""
+    wt, A = _problem(M, N, K, 128, 31 + M)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    assert marlin.plan_2_4(M, K, N)["splits"] > 1 and marlin.plan_2_4(M, K, N, noalloc=True)["splits"] == 1
+    warm, cold = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(warm):
+        C0 = torch.empty(M, N, dtype=torch.half, device=DEV)
+        marlin.mul_2_4(A, wt["B"], wt["meta"], C0, wt["s"], ws)
+    torch.cuda.synchronize()
+    C1 = torch.empty_like(C0)
+    marlin.mul_2_4_noalloc(A, wt["B"], wt["meta"], C1, wt["s"])
+    assert_close(C1.cpu().numpy(), C0.cpu().numpy(), "no-allocation call")
+    for s, ref in ((warm, C0), (cold, None)):
+        C = torch.zeros_like(C0)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            marlin.mul_2_4(A, wt["B"], wt["meta"], C, wt["s"], ws)
+        for _ in range(3):
+            C.fill_(float("nan"))
+            marlin.mul_2_4(A, wt["B"], wt["meta"], C1, wt["s"], ws)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            if ref is not None:
+                assert torch.equal(C, ref)
+            else:
+                assert_close(C.cpu().numpy(), C0.cpu().numpy(), "captured without scratch")
+
+
+@pytest.mark.parametrize("M,N,K,g", [(129, 16384, 1152, 128), (96, 22016, 1024, -1), (150, 12288, 2176, 128),
+                                     (192, 22016, 1024, 128), (129, 2048, 28672, 128), (100, 2816, 17408, -1)])
 def test_prefill_two_group_tiles(M, N, K, g):
     """Two k-groups per workgroup (65-192 rows, K from 1024): 64- and 96-row tiles,
     equal and unequal shares of the k-steps (K = 1152: 4 and 5 pairs), ragged rows,

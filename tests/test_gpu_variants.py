@@ -132,6 +132,32 @@ def test_w3_gemm_bit_exact_against_4bit_path(M, K, N):
     assert torch.equal(C3, C4)
 
 
+MID_CASES = [(64, 4096, 22016), (48, 4096, 4096), (131, 4096, 4096), (96, 2048, 10240), (80, 1024, 12288),
+             (40, 8192, 10240)]
+
+
+@pytest.mark.parametrize("M,K,N", MID_CASES)
+def test_mid_batches_3bit(M, K, N):
+    """The mid-batch kernel (33-192 rows) on 3-bit metadata and 3-bit values: the same
+    tiles and order of sums as 4-bit operands, so bit-identical to the 4-bit calls."""
+    assert marlin.plan_2_4(M, K, N)["threads"] == 512
+    A = synth.make_activation(M, K, 7 + M, device=DEV)
+
+    def run(fn, B, meta, s):
+        C = torch.full((M, N), float("nan"), dtype=torch.half, device=DEV)
+        fn(A, B, meta, C, s, _ws(N))
+        torch.cuda.synchronize()
+        return C
+
+    wt = synth.make_weight(K, N, 41 + M, 128, device=DEV)
+    ref = run(marlin.mul_2_4, wt["B"], wt["meta"], wt["s"])
+    assert torch.isfinite(ref).all()
+    assert torch.equal(run(marlin.mul_2_4_meta3, wt["B"], marlin.pack_meta3(wt["meta"]), wt["s"]), ref)
+    w3 = synth.make_weight(K, N, 43 + M, 128, bits=3, device=DEV)
+    C3 = run(marlin.mul_2_4_w3, w3["B"], w3["meta"], w3["s"])
+    assert torch.equal(run(marlin.mul_2_4, _w3_as_w4(w3["B"]), w3["meta"], w3["s"]), C3)
+
+
 # Shapes that the decode tile table sends to the 8-row batch at 5-8 rows (activations
 # staged through LDS): 4096x4096 on 16-column tiles of 8 waves, 4096x22016 at M = 5 on
 # 32-column tiles, 8192x57344 on 64-column tiles.
