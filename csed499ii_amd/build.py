@@ -56,7 +56,7 @@ _PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
 EXTRA_FLAGS: dict[str, list[str]] = {
     name: _PRELOAD for name in ("sm24_decode_16.hip", "sm24_decode_32.hip", "sm24_decode_64.hip", "sm24_mid.hip",
                                 "sm24_mid_w3.hip", "sm24_mid_m3.hip", "sm24_gemm.hip",
-                                "marlin_dense.hip")}
+                                "marlin_dense.hip", "marlin_dense_mid.hip")}
 
 # hipcc's host pass does not know the packed-fp32 target feature: drop that noise.
 _NOISE = ("packed-fp32-ops", "is not a recognized feature")

@@ -20,11 +20,11 @@
 // nibbles).  So one lane loads the two 16-byte word groups (ci, rq, jt = 0..3) and
 // feeds the four column tiles of the chunk from them.
 //
-// Work decomposition (one launch): grid.x 64-column chunk, grid.y K split, grid.z
-// batch tile of 16*BB rows; NW waves take contiguous ranges of the split's k-steps
-// through a ring of U in-flight fragments and are reduced in LDS in a fixed order;
-// with several splits the last workgroup to arrive at the tile's counter adds the
-// splits' fp32 partials in split order (bit-identical from run to run).
+// Three kernels.  Up to 2048 rows mostly marlin_dense_mid.h, above that (and for much
+// work) marlin_dense_prefill.h.  The kernel here takes what neither covers: activations of 4 GiB
+// and more (their kernels address them by 32-bit offsets).  Its work decomposition: grid.x
+// 64-column chunk, grid.z batch tile of 64 rows; NW waves take contiguous ranges of the
+// k-steps through a ring of U in-flight fragments and are reduced in LDS in a fixed order.
 //
 // Reference: marlin_cuda_kernel.cu (Marlin at 90-605, host dispatch marlin_cuda at
 // 655-736) and marlin_cuda.cpp:38-64 (the binding's checks).
@@ -32,6 +32,7 @@
 #include <stdint.h>
 #include <stdlib.h>
 
+#include "marlin_dense_mid.h"
 #include "marlin_dense_prefill.h"
 #include "sm24_device.h"
 #include "sm24_host.h"
@@ -46,12 +47,11 @@ struct DenseArgs {
   _Float16* C;
   const _Float16* zeros;  // >= 64 zero bytes (rows past M)
   int M, N, K;
-  int splits;
-  float* partial;      // [splits][M][N] when splits > 1
-  uint32_t* counters;  // [gridDim.z][gridDim.x], zero between launches
 };
 
-template <int BB, bool GROUPED>
+constexpr int BB = 4;  // 16-row blocks per batch tile
+
+template <bool GROUPED>
 struct DenseFrag {
   u32x4 w0, w1;      // word groups (ci, rq0, jt = 0..3) and (ci, rq0 + 1, jt = 0..3)
   half8_t sc;        // grouped: scale slots 8*ci .. 8*ci + 7 (columns ci + 8j)
@@ -62,9 +62,9 @@ struct DenseFrag {
 // into SGPRs (this translation unit is built with -mllvm
 // -amdgpu-kernarg-preload-count=14), ahead of the whole DenseArgs; the fp16
 // pointers travel as void pointers, which keeps the kernel's name demangleable.
-template <int BB, int NW, bool GROUPED>
+template <int NW, bool GROUPED>
 __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, const uint32_t* B_, const void* s_,
-                                                               const void* zeros_, int M_, int N_, int K_, int splits_,
+                                                               const void* zeros_, int M_, int N_, int K_, int nks_,
                                                                DenseArgs a_) {
   DenseArgs a = a_;
   a.A = static_cast<const _Float16*>(A_);
@@ -74,18 +74,11 @@ __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, c
   a.M = M_;
   a.N = N_;
   a.K = K_;
-  a.splits = splits_;
   constexpr int NT = 64 * NW;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int chunk = blockIdx.x, split = blockIdx.y, bt = blockIdx.z;
+  const int chunk = blockIdx.x, bt = blockIdx.z;
   const int N = a.N, K = a.K, M = a.M;
-  const int nks = K >> 5;  // 32-deep k-steps
-  int ks0 = 0, ks1 = nks;
-  if (a.splits > 1) {  // uniform; nks * splits is small, so 32 bits are exact
-    ks0 = (int)((unsigned)(nks * split) / (unsigned)a.splits);
-    ks1 = (int)((unsigned)(nks * (split + 1)) / (unsigned)a.splits);
-  }
   const int h = lane >> 4, rho = lane & 15;
   const int ci = rho & 7, b = rho >> 3;
   const int kt = h >> 1, rq0 = 2 * (h & 1);
@@ -98,7 +91,7 @@ __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, c
   const int row0 = 16 * BB * bt + rho;
   const int koff = 16 * kt + 4 * (h & 1);
 
-  auto fetch = [&](int ks, bool live, DenseFrag<BB, GROUPED>& f) {
+  auto fetch = [&](int ks, bool live, DenseFrag<GROUPED>& f) {
     const uint32_t* p = bw + (size_t)ks * bstep;
     f.w0 = *reinterpret_cast<const u32x4*>(p);
     f.w1 = *reinterpret_cast<const u32x4*>(p + 4);
@@ -127,7 +120,7 @@ __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, c
   asm volatile("v_mov_b32 %0, 0x00f000f0" : "=v"(kMaskHi));
   asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(kMagic));
   const uint32_t ssh = 16u * (uint32_t)b;  // the lane's scale: half b of scale word jt
-  auto compute = [&](const DenseFrag<BB, GROUPED>& f) {
+  auto compute = [&](const DenseFrag<GROUPED>& f) {
 #pragma unroll
     for (int jt = 0; jt < 4; jt++) {
       // column 16 jt + rho: byte b of words rq0 (k 4(h&1) + 0, 1 | 8 + ...) and rq0 + 1;
@@ -156,13 +149,11 @@ __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, c
 
   // Each wave streams a contiguous share of the split's k-steps through a ring of U
   // fragments; slots past the end re-read the last k-step with zero activations.
-  constexpr int U = BB == 1 ? 6 : 4;
-  const int span = ks1 - ks0;
-  const int r0 = ks0 + span * wave / NW;
-  const int r1 = ks0 + span * (wave + 1) / NW;
+  constexpr int U = 4;
+  const int r0 = nks_ * wave / NW, r1 = nks_ * (wave + 1) / NW;  // 32-deep k-steps
   if (r1 > r0) {
     const int rlast = r1 - 1;
-    DenseFrag<BB, GROUPED> ring[U];
+    DenseFrag<GROUPED> ring[U];
 #pragma unroll
     for (int i = 0; i < U; i++) {
       fetch(r0 + i < r1 ? r0 + i : rlast, r0 + i < r1, ring[i]);
@@ -199,25 +190,6 @@ __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, c
     const int c = nl & 31;
     return a.s[ncol0 + (nl & 32) + 8 * ((c & 7) >> 1) + 2 * (c >> 3) + (c & 1)];
   };
-  if (a.splits == 1) {
-    for (int e = threadIdx.x; e < ntile; e += NT) {
-      const int ml = e >> 6, nl = e & 63;
-      const int m = 16 * BB * bt + ml;
-      if (m >= M) continue;
-      float v = red[0][ml][nl];
-#pragma unroll
-      for (int w = 1; w < NW; w++) v += red[w][ml][nl];
-      _Float16 o = (_Float16)v;
-      if constexpr (!GROUPED) o = o * col_scale(nl);
-      a.C[(size_t)m * N + ncol0 + nl] = o;
-    }
-    return;
-  }
-
-  // Split-K hand-off through the uncached scratch (device-scope atomic accesses): each
-  // thread's partial stores complete before the workgroup barrier, the tile's counter
-  // is bumped after it, and the last split to arrive adds all partials in split order,
-  // writes C and resets the counter.
   for (int e = threadIdx.x; e < ntile; e += NT) {
     const int ml = e >> 6, nl = e & 63;
     const int m = 16 * BB * bt + ml;
@@ -225,42 +197,10 @@ __global__ __launch_bounds__(64 * NW) void marlin_dense_kernel(const void* A_, c
     float v = red[0][ml][nl];
 #pragma unroll
     for (int w = 1; w < NW; w++) v += red[w][ml][nl];
-    __hip_atomic_store(a.partial + ((size_t)split * M + m) * N + ncol0 + nl, v, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0);
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __syncthreads();
-  __shared__ uint32_t arrived;
-  uint32_t* cnt = a.counters + bt * gridDim.x + chunk;
-  if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-  __syncthreads();
-  if (arrived != (uint32_t)a.splits) return;
-  for (int e = threadIdx.x; e < ntile; e += NT) {
-    const int ml = e >> 6, nl = e & 63;
-    const int m = 16 * BB * bt + ml;
-    if (m >= M) continue;
-    const float* pp = a.partial + (size_t)m * N + ncol0 + nl;
-    const size_t pstride = (size_t)M * N;
-    float v = 0.f;
-    int q = 0;
-    for (; q + 4 <= a.splits; q += 4) {  // four loads in flight, summed in split order
-      const float p0 = __hip_atomic_load(pp + (q + 0) * pstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float p1 = __hip_atomic_load(pp + (q + 1) * pstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float p2 = __hip_atomic_load(pp + (q + 2) * pstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float p3 = __hip_atomic_load(pp + (q + 3) * pstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      v += p0;
-      v += p1;
-      v += p2;
-      v += p3;
-    }
-    for (; q < a.splits; q++) v += __hip_atomic_load(pp + q * pstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     _Float16 o = (_Float16)v;
     if constexpr (!GROUPED) o = o * col_scale(nl);
     a.C[(size_t)m * N + ncol0 + nl] = o;
   }
-  if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------
@@ -292,49 +232,18 @@ int dense_validate(int prob_m, int prob_n, int prob_k, int groupsize, int thread
   return MARLIN_HIP_OK;
 }
 
-template <int BB, bool G>
+template <bool G>
 hipError_t launch_dense_t(const DenseArgs& a, dim3 grid, hipStream_t stream) {
   constexpr int NW = 4;
-  hipLaunchKernelGGL((marlin_dense_kernel<BB, NW, G>), grid, dim3(64 * NW), 0, stream, a.A, a.B, a.s, a.zeros, a.M,
-                     a.N, a.K, a.splits, a);
+  hipLaunchKernelGGL((marlin_dense_kernel<NW, G>), grid, dim3(64 * NW), 0, stream, a.A, a.B, a.s, a.zeros, a.M, a.N,
+                     a.K, a.K / 32, a);
   return hipGetLastError();
 }
 
-// K splits, from forced splits 1-16 over the Llama-2-7B decode calls (MI355X): a
-// split's hand-off costs microseconds, so tiles that already cover at least 3/4 of
-// the CUs run unsplit (qkv, 192 chunks: 16.0 -> 13.8 us at M = 1 against three
-// splits); fewer tiles split to about one workgroup per CU (o and down, 64 chunks:
-// four splits, 9.9 -> 9.0 and 12.7 -> 12.2 us against eight); between one and two
-// tiles per CU split in two, which balances the CUs (gate_up, 344 chunks: 20.7
-// against 22.3 us unsplit).  Each wave keeps at least two k-steps; at most 16
-// splits and one arrival counter per (chunk, batch tile).  MARLIN_HIP_DENSE_SPLITS
-// forces the count.
-int dense_splits(int chunks, int ztiles, int nks, int cus) {
-  static const int forced = [] {
-    const char* e = getenv("MARLIN_HIP_DENSE_SPLITS");
-    const int x = e ? atoi(e) : 0;
-    return x >= 1 && x <= 16 ? x : 0;
-  }();
-  const long long tiles = (long long)chunks * ztiles;
-  int s = 1;
-  if (forced) s = forced;
-  else if (tiles >= cus) s = tiles < 2LL * cus ? 2 : 1;
-  else if (4 * tiles < 3LL * cus) s = (int)((cus + tiles / 2) / tiles);
-  const int smax = nks / 8 > 0 ? nks / 8 : 1;
-  if (s > smax) s = smax;
-  if (s > 16) s = 16;
-  if (s < 1) s = 1;
-  if ((size_t)tiles * sizeof(uint32_t) > kCounterBytes) s = 1;
-  return s;
-}
-
 // Large-M path (marlin_dense_prefill_kernel): K a multiple of 128 (whole scale groups, an
-// even number of 64-deep k-steps), N of its 512-column tile, or of half of it (the last
-// tile is then half empty) where that beats the decode-shaped kernel: from 4096 columns,
-// and above 512 rows (us per call, one box: 4096x11008 at M = 65 / 200 / 777 50.8 / 104 /
-// 309 -> 38.2 / 48.4 / 92.7; 4096x2816 at M = 777 / 2000 107 / 208 -> 51.5 / 83.4, but at
-// M = 300 37.4 against 43.3).  32-bit operand offsets; from
-// MARLIN_HIP_DENSE_PREFILL_MIN_M rows (default 65).
+// even number of 64-deep k-steps), N of its 512-column tile or of half of it (the last tile
+// is then half empty).  32-bit operand offsets; from MARLIN_HIP_DENSE_PREFILL_MIN_M rows
+// (default 65).
 bool dense_prefill_fits(int M, int N, int K) {
   static const int forced_min_m = [] {
     const char* e = getenv("MARLIN_HIP_DENSE_PREFILL_MIN_M");
@@ -342,8 +251,7 @@ bool dense_prefill_fits(int M, int N, int K) {
     return x >= 1 ? x : 0;
   }();
   const int min_m = forced_min_m ? forced_min_m : 65;
-  const bool cols = N % kDpTileCols == 0 || (N % (kDpTileCols / 2) == 0 && (N >= 4096 || M > 512));
-  return M >= min_m && cols && K % 128 == 0 && (long long)M * K < (1LL << 31) - 2048 &&
+  return M >= min_m && N % (kDpTileCols / 2) == 0 && K % 128 == 0 && (long long)M * K < (1LL << 31) - 2048 &&
          (long long)K * N < (1LL << 33);
 }
 
@@ -351,8 +259,8 @@ bool dense_prefill_fits(int M, int N, int K) {
 // one workgroup per CU times the k-steps per split, plus the partial exchange (each
 // split stores a 256 KiB fp32 tile), at ~1.3 us per 64-deep k-step of a tile (32
 // MFMAs per wave) and ~2.5 TB/s for the exchange.  MARLIN_HIP_DENSE_PREFILL_SPLITS
-// forces a count.
-int dense_prefill_splits(int tiles, int nks, int cus) {
+// forces a count.  *estimate: the model's time, us.
+int dense_prefill_splits(int tiles, int nks, int cus, double* estimate = nullptr) {
   static const int forced = [] {
     const char* e = getenv("MARLIN_HIP_DENSE_PREFILL_SPLITS");
     const int x = e ? atoi(e) : 0;
@@ -373,6 +281,7 @@ int dense_prefill_splits(int tiles, int nks, int cus) {
     }
   }
   if ((size_t)tiles * sizeof(uint32_t) > kCounterBytes) best_s = 1;
+  if (estimate) *estimate = best;
   return best_s;
 }
 
@@ -396,6 +305,82 @@ int run_dense_prefill(const void* A, const void* B, void* C, const void* s, int 
   return launch_error(launch_dense_prefill(p, grouped, stream));
 }
 
+// Tile and K splits of the decode- and mid-batch kernel (marlin_dense_mid.h), from a cost
+// model fitted to 1000 forced plans (every tile x splits 1-8 on twelve K x N, 1024x5120 to
+// 28672x8192, M from 1 to 512, one box; mean error 5 %, the model's choices 1.5 % from the
+// best of each call): a fixed cost, the stages of a wave at the tile's measured stage time
+// per round of workgroups over the CUs (16-row tiles run two workgroups per CU), the
+// reduction in LDS, the codes' bytes, and for a split the exchange of the fp32 partials
+// (only up to one workgroup per CU).  *cost in us.
+DenseMidShape dense_mid_plan(int M, int N, int K, int cus, bool nosplit, double* cost) {
+  struct Cand {
+    int nch, rb;
+    double stage_us;
+  };
+  static const Cand cands[] = {{1, 1, 0.64}, {1, 2, 0.86}, {1, 3, 1.00}, {1, 4, 1.06}, {1, 5, 1.26},
+                               {2, 1, 1.05}, {2, 2, 1.35}, {2, 3, 1.48}, {2, 4, 1.70}};
+  DenseMidShape best{1, 1, 1};
+  double best_cost = 1e30;
+  for (const Cand& c : cands) {
+    if (N % (64 * c.nch) != 0) continue;
+    const long long tiles = (long long)(N / (64 * c.nch)) * ((M + 16 * c.rb - 1) / (16 * c.rb));
+    for (int s = 1; s <= (nosplit ? 1 : 8); s++) {
+      if (s > 1 && (tiles * s > cus || K / 64 < 8 * s)) break;
+      const double x = (double)(tiles * s) / cus;
+      const double rounds = x <= 1 ? 1 : (double)((tiles * s + cus - 1) / cus);
+      const double f = x > 1 && c.rb == 1 ? 1.3 * x : rounds * (1 + 0.29 * (x / rounds - 0.75));
+      double t = 2.7 + (K / 64 / s + 7) / 8 * c.stage_us * f + 0.49 * c.nch * c.rb * rounds + 2.4e-8 * K * (double)N;
+      if (s > 1) t += 1.4 + 8.0 * s * M * (double)N / 7.65e6;
+      if (t < best_cost) {
+        best_cost = t;
+        best = DenseMidShape{c.nch, c.rb, s};
+      }
+    }
+  }
+  if (cost) *cost = best_cost;
+  return best;
+}
+
+// Whether a call runs the decode- and mid-batch kernel: up to 64 rows always, up to 2048
+// where the large-M kernel does not take the shape or its own planner's estimate is not
+// clearly lower.  Over the sweep above and 90 random shapes at 400-4096 rows this keeps
+// the faster of the two or one within a few per cent of it up to 2048 rows (large-M ->
+// this kernel, us: 943x1792x3584 43.7 -> 28.0, 768x11008x1536 68.1 -> 36.9, 1168x1280x1280
+// 34.3 -> 12.2); beyond, two calls lost (3257x10752x2560 201.9 -> 224.3).  32-bit
+// activation offsets.
+constexpr int kDenseMidMaxM = 2048;
+bool dense_mid_fits(int M, int N, int K, int cus) {
+  if (M > kDenseMidMaxM || (long long)M * K >= (1LL << 31)) return false;
+  if (!dense_prefill_fits(M, N, K)) return true;
+  const int tiles = ((N + kDpTileCols - 1) / kDpTileCols) * ((M + kDpRows - 1) / kDpRows);
+  double mid = 0.0, pre = 0.0;
+  dense_mid_plan(M, N, K, cus, false, &mid);
+  dense_prefill_splits(tiles, K / 64, cus, &pre);
+  return mid < 0.82 * (pre + 6.0);
+}
+
+int run_dense_mid(const void* A, const void* B, void* C, const void* s, int M, int N, int K, bool grouped, int dev,
+                  hipStream_t stream, int sms) {
+  DensePreArgs p{};
+  p.A = static_cast<const _Float16*>(A);
+  p.B = static_cast<const uint32_t*>(B);
+  p.s = static_cast<const _Float16*>(s);
+  p.C = static_cast<_Float16*>(C);
+  p.M = M;
+  p.N = N;
+  p.K = K;
+  DenseMidShape d = dense_mid_plan(M, N, K, sms, false, nullptr);
+  if (d.splits > 1) {
+    const size_t tiles = (size_t)(N / (64 * d.nch)) * ((M + 16 * d.rb - 1) / (16 * d.rb));
+    const int err =
+        get_scratch(dev, stream, tiles * d.splits * 1024 * d.nch * d.rb * sizeof(float), &p.counters, &p.partial);
+    if (err != MARLIN_HIP_OK) return err;
+    if (!p.counters) d = dense_mid_plan(M, N, K, sms, true, nullptr);  // capturing, no scratch yet
+  }
+  p.splits = d.splits;
+  return launch_error(launch_dense_mid(p, d, grouped, stream));
+}
+
 int run_dense(const void* A, const void* B, void* C, const void* s, int prob_m, int prob_n, int prob_k,
               int groupsize, int dev, hipStream_t stream, int thread_k, int thread_n, int sms) {
   int err = dense_validate(prob_m, prob_n, prob_k, groupsize, thread_k, thread_n);
@@ -412,9 +397,9 @@ int run_dense(const void* A, const void* B, void* C, const void* s, int prob_m, 
     if (hipDeviceGetAttribute(&sms, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || sms <= 0)
       sms = 256;
   }
+  if (dense_mid_fits(M, N, K, sms)) return run_dense_mid(A, B, C, s, M, N, K, groupsize != -1, dev, stream, sms);
   if (dense_prefill_fits(M, N, K)) return run_dense_prefill(A, B, C, s, M, N, K, groupsize != -1, dev, stream, sms);
-  const int bb = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  const int ztiles = (M + 16 * bb - 1) / (16 * bb);
+  const int ztiles = (M + 16 * BB - 1) / (16 * BB);
   const int chunks = N / 64;
   DenseArgs a{};
   a.A = static_cast<const _Float16*>(A);
@@ -426,19 +411,8 @@ int run_dense(const void* A, const void* B, void* C, const void* s, int prob_m, 
   a.K = K;
   err = get_zeros(dev, stream, &a.zeros);
   if (err != MARLIN_HIP_OK) return err;
-  a.splits = dense_splits(chunks, ztiles, K / 32, sms);
-  if (a.splits > 1) {
-    err = get_scratch(dev, stream, (size_t)a.splits * M * N * sizeof(float), &a.counters, &a.partial);
-    if (err != MARLIN_HIP_OK) return err;
-    if (!a.counters) a.splits = 1;  // capturing, and this stream has no scratch yet
-  }
-  const dim3 grid(chunks, a.splits, ztiles);
-  const bool grouped = groupsize != -1;
-  hipError_t e;
-  if (bb == 1) e = grouped ? launch_dense_t<1, true>(a, grid, stream) : launch_dense_t<1, false>(a, grid, stream);
-  else if (bb == 2) e = grouped ? launch_dense_t<2, true>(a, grid, stream) : launch_dense_t<2, false>(a, grid, stream);
-  else e = grouped ? launch_dense_t<4, true>(a, grid, stream) : launch_dense_t<4, false>(a, grid, stream);
-  return launch_error(e);
+  const dim3 grid(chunks, 1, ztiles);
+  return launch_error(groupsize != -1 ? launch_dense_t<true>(a, grid, stream) : launch_dense_t<false>(a, grid, stream));
 }
 
 }  // namespace sm24

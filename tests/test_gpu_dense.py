@@ -148,6 +148,70 @@ def test_dense_reference_bench_call_site(m, k, n):
         assert_close(C[:, 64 * c0:64 * (c0 + 2)].cpu().numpy(), _oracle(A, wt, c0, 2), f"dense bench {m}x{k}x{n}")
 
 
+# ---- the decode- and mid-batch kernel (marlin_dense_mid_kernel) ----
+
+@pytest.mark.parametrize("M,N,K,g", [(1, 128, 128, -1), (5, 256, 1152, 128), (8, 4096, 4096, 128),
+                                     (9, 12288, 1024, -1), (16, 22016, 512, 128), (17, 2048, 2048, 128),
+                                     (33, 256, 128, -1), (48, 5120, 1024, 128), (64, 11008, 1024, -1),
+                                     (80, 12288, 1024, 128), (96, 4096, 4096, 128), (131, 2048, 8192, 128),
+                                     (160, 22016, 256, 128), (200, 4096, 1024, -1), (300, 1280, 640, 128),
+                                     (512, 2048, 1024, 128), (1100, 1280, 1280, -1)])
+def test_dense_mid_batches(M, N, K, g):
+    """Every tile the planner gives (64 and 128 columns, 16 to 80 rows, one activation
+    instruction up to 8 rows), fewer k-steps than waves (K = 128), shares that do not
+    divide (K = 640, 1152), K splits handed off through the scratch, several rounds of
+    workgroups: column slices against the oracle, nothing past C's end, repeated calls
+    bit-identical."""
+    wt = _dense_weight(K, N, g, 7 * M + N + K)
+    A = synth.make_activation(M, K, M + 17, device=DEV)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C = buf[:M * N].view(M, N)
+    ws = torch.zeros(max(N // 128 * 16, 16), dtype=torch.int32, device=DEV)
+    marlin.mul(A, wt["B"], C, wt["s"], ws)
+    torch.cuda.synchronize()
+    assert torch.isfinite(C).all() and bool((buf[M * N:] == 7.0).all())
+    chunks = N // 64
+    for c0 in sorted({0, max(chunks // 2 - 1, 0), chunks - 2}):
+        assert_close(C[:, 64 * c0:64 * (c0 + 2)].cpu().numpy(), _oracle(A, wt, c0, 2),
+                     f"dense mid M={M} N={N} K={K} g={g} chunk {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(A, wt), C), "repeated calls differ"
+
+
+def test_dense_mid_capture_without_scratch():
+    """A call whose plan splits K (4096x4096 at 8 rows), captured on a stream that has no
+    scratch yet, runs unsplit: the eager result within the GEMM tolerance, on every replay."""
+    wt = _dense_weight(4096, 4096, 128, 21)
+    A = synth.make_activation(8, 4096, 22, device=DEV)
+    ref = _run(A, wt)
+    ws = torch.zeros(512, dtype=torch.int32, device=DEV)
+    C = torch.zeros(8, 4096, dtype=torch.half, device=DEV)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        marlin.mul(A, wt["B"], C, wt["s"], ws)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        assert torch.equal(_run(A, wt), ref)
+        g.replay()
+        torch.cuda.synchronize()
+        assert_close(C.cpu().numpy(), ref.cpu().numpy(), "captured without scratch")
+
+
+def test_dense_activations_beyond_32_bit_offsets():
+    """M K of 2^31 and more (4 GiB of activations) runs the multi-block kernel: rows at
+    the start, in the middle and at the end against the same rows as small calls."""
+    K, N = 28672, 256
+    M = (1 << 31) // K + 70
+    wt = _dense_weight(K, N, 128, 23)
+    gen = torch.Generator(device=DEV).manual_seed(24)
+    A = torch.randn((M, K), dtype=torch.half, device=DEV, generator=gen)
+    C = _run(A, wt)
+    assert torch.isfinite(C).all()
+    for r0 in (0, M // 2, M - 16):
+        part = _run(A[r0:r0 + 16].contiguous(), wt)
+        assert_close(C[r0:r0 + 16].cpu().numpy(), part.cpu().numpy(), f"rows {r0}")
+
+
 # ---- large batches: the MFMA-bound dense kernel (marlin_dense_prefill_kernel) ----
 
 @pytest.mark.parametrize("M,N,K,g", [(65, 512, 128, 128), (128, 512, 1024, -1), (300, 1024, 2048, 128),
@@ -167,8 +231,8 @@ def test_dense_large_m_against_oracle(M, N, K, g):
     assert torch.equal(_run(A, wt), C), "repeated dense large-M calls differ"
 
 
-@pytest.mark.parametrize("M,N,K,g", [(65, 4352, 128, 128), (130, 4352, 2048, -1), (520, 768, 4096, 128),
-                                     (513, 256, 256, -1)])
+@pytest.mark.parametrize("M,N,K,g", [(2100, 768, 1024, 128), (2049, 256, 256, -1), (1500, 4864, 4096, 128),
+                                     (520, 768, 4096, 128)])
 def test_dense_large_m_ragged_columns(M, N, K, g):
     """N a multiple of 256 but not of the 512-column tile (the last tile's upper four
     waves store nothing): all columns against the oracle, nothing past C's end, and
