@@ -306,19 +306,19 @@ int run_dense_prefill(const void* A, const void* B, void* C, const void* s, int 
 }
 
 // Tile and K splits of the decode- and mid-batch kernel (marlin_dense_mid.h), from a cost
-// model fitted to 1000 forced plans (every tile x splits 1-8 on twelve K x N, 1024x5120 to
-// 28672x8192, M from 1 to 512, one box; mean error 5 %, the model's choices 1.5 % from the
+// model fitted to 2000 forced plans (every tile x splits 1-8 on eleven K x N, 1024x5120 to
+// 8192x57344, M from 1 to 512, one box; mean error 5 %, the model's choices 0.6 % from the
 // best of each call): a fixed cost, the stages of a wave at the tile's measured stage time
-// per round of workgroups over the CUs (16-row tiles run two workgroups per CU), the
-// reduction in LDS, the codes' bytes, and for a split the exchange of the fp32 partials
+// per round of workgroups over the CUs (less for the small tiles, two of which share a CU),
+// the reduction in LDS, the codes' bytes, and for a split the exchange of the fp32 partials
 // (only up to one workgroup per CU).  *cost in us.
 DenseMidShape dense_mid_plan(int M, int N, int K, int cus, bool nosplit, double* cost) {
   struct Cand {
     int nch, rb;
     double stage_us;
   };
-  static const Cand cands[] = {{1, 1, 0.64}, {1, 2, 0.86}, {1, 3, 1.00}, {1, 4, 1.06}, {1, 5, 1.26},
-                               {2, 1, 1.05}, {2, 2, 1.35}, {2, 3, 1.48}, {2, 4, 1.70}};
+  static const Cand cands[] = {{1, 1, 0.60}, {1, 2, 0.72}, {1, 3, 0.92}, {1, 4, 1.06}, {1, 5, 1.26},
+                               {2, 1, 1.07}, {2, 2, 1.27}, {2, 3, 1.51}, {2, 4, 1.73}};
   DenseMidShape best{1, 1, 1};
   double best_cost = 1e30;
   for (const Cand& c : cands) {
@@ -328,9 +328,10 @@ DenseMidShape dense_mid_plan(int M, int N, int K, int cus, bool nosplit, double*
       if (s > 1 && (tiles * s > cus || K / 64 < 8 * s)) break;
       const double x = (double)(tiles * s) / cus;
       const double rounds = x <= 1 ? 1 : (double)((tiles * s + cus - 1) / cus);
-      const double f = x > 1 && c.rb == 1 ? 1.3 * x : rounds * (1 + 0.29 * (x / rounds - 0.75));
-      double t = 2.7 + (K / 64 / s + 7) / 8 * c.stage_us * f + 0.49 * c.nch * c.rb * rounds + 2.4e-8 * K * (double)N;
-      if (s > 1) t += 1.4 + 8.0 * s * M * (double)N / 7.65e6;
+      const double share = x > 1 && c.nch * c.rb <= 2 ? 0.89 : 1.0;
+      const double f = share * rounds * (1 + 0.295 * (x / rounds - 0.75));
+      double t = 2.7 + (K / 64 / s + 7) / 8 * c.stage_us * f + 0.50 * c.nch * c.rb * rounds + 2.8e-8 * K * (double)N;
+      if (s > 1) t += 1.44 + 8.0 * s * M * (double)N / 7.5e6;
       if (t < best_cost) {
         best_cost = t;
         best = DenseMidShape{c.nch, c.rb, s};

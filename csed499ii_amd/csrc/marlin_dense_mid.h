@@ -11,15 +11,15 @@
 // activation rows (L2 hits: 128 bytes per row and k-step against 33 per column) on the
 // 64-byte-per-clock path into the compute unit, and the latency of both.  All operands
 // come by LDS-DMA (codes 1 KiB to an instruction, activation rows in whole 128-byte
-// lines) into rings that take the whole LDS (half of it for 16-row tiles: two workgroups
-// per CU), and a stage's buffer is refilled as soon as the stage is in registers.  The
-// kernel this replaces loaded 8 bytes per lane straight into operand order, through the
-// same path 64 lanes at a time, and re-read the codes for every 64 rows.
+// lines) into one stage buffer per wave, refilled as soon as the stage is in registers
+// (buffers for more stages were no faster: see sm24_mid.h).  The kernel this replaces
+// loaded 8 bytes per lane straight into operand order, through the same path 64 lanes at
+// a time, and re-read the codes for every 64 rows.
 //
 // us per call, the kernels before -> this one (one box): 7B at M = 4 qkv 12.4 -> 9.0, o
-// 8.6 -> 7.0, gate_up 22.4 -> 13.7, down 11.8 -> 9.6; M = 64 38.3 -> 15.8, 22.1 -> 9.0,
-// 69.3 -> 23.3, 36.7 -> 15.4; against the large-M kernel at M = 131 48.6 -> 31.3, 42.5 ->
-// 11.5, 65.6 -> 48.9, 61.5 -> 24.6, at M = 512 4096x4096 45.9 -> 22.0, 2048x2048 35.1 ->
+// 8.6 -> 6.8, gate_up 22.4 -> 13.3, down 11.8 -> 9.6; M = 64 38.3 -> 15.6, 22.1 -> 8.3,
+// 69.3 -> 23.1, 36.7 -> 15.0; against the large-M kernel at M = 131 48.6 -> 29.3, 42.5 ->
+// 10.4, 65.6 -> 46.5, 61.5 -> 24.0, at M = 512 4096x4096 45.9 -> 22.0, 2048x2048 35.1 ->
 // 8.7; 70B down 28672x8192 at M = 1 37.2 -> 25.9.
 #pragma once
 #include "marlin_dense_prefill.h"
@@ -29,21 +29,19 @@ namespace sm24 {
 
 constexpr int kDmWaves = 8;
 
-// One wave's ring: D stages of its own activation rows, codes and scales; the
-// workgroup's reduction buffer lies in the same space.  AI: activation DMAs per stage (8
-// rows each).
-template <int NCH, int RB, int AI, bool GROUPED>
+// One wave's stage buffer (its activation rows, codes and scales of one k-step); the
+// workgroup's reduction buffer lies in the same space.
+template <int NCH, int RB, bool GROUPED>
 struct DmLds {
   static constexpr int TC = 64 * NCH;
   static constexpr int act_b = 16 * RB * 128;       // activation rows of one 64-deep k-step
   static constexpr int stage_b = act_b + NCH * (2048 + (GROUPED ? 128 : 0));
-  static constexpr int L = AI + NCH * 2 + (GROUPED ? 1 : 0);  // DMA instructions per stage
-  static constexpr int lds = (RB == 1 ? 80 : 160) * 1024;
-  static constexpr int D = cmin(4, cmin(lds / (kDmWaves * stage_b), 60 / L + 1));
   static constexpr int redp = TC + 4;               // floats of one reduction row
   static constexpr int red_row = kDmWaves * 16 * redp * 4;  // 16 rows of every wave
-  static constexpr int RC = cmin(RB, 160 * 1024 / red_row);  // 16-row blocks reduced at a time
-  static constexpr int bytes = cmax(D * kDmWaves * stage_b, RC * red_row);
+  // 16-row blocks reduced at a time: half the LDS where the registers let two workgroups
+  // share a compute unit
+  static constexpr int RC = cmin(RB, (4 * NCH * RB <= 12 ? 80 : 160) * 1024 / red_row);
+  static constexpr int bytes = cmax(kDmWaves * stage_b, RC * red_row);
 };
 
 template <int NCH, int RB, int AI, bool GROUPED>
@@ -55,10 +53,10 @@ __global__ __launch_bounds__(64 * kDmWaves) void marlin_dense_mid_kernel(const v
   // the fp16 pointers travel as void pointers, which keeps the kernel's name demangleable
   const DensePreArgs a{static_cast<const _Float16*>(A_), B_, static_cast<const _Float16*>(s_),
                        static_cast<_Float16*>(C_), M_, N_, K_, splits_, partial_, counters_};
-  using T = DmLds<NCH, RB, AI, GROUPED>;
-  constexpr int D = T::D, L = T::L, MB = 16 * RB, TC = T::TC, KG = kDmWaves, NT = 4 * NCH;
+  using T = DmLds<NCH, RB, GROUPED>;
+  constexpr int MB = 16 * RB, TC = T::TC, KG = kDmWaves, NT = 4 * NCH;
   constexpr int WOFF = T::act_b, SOFF = WOFF + 2048 * NCH;
-  static_assert(D >= 1 && (AI == 2 * RB || (RB == 1 && AI == 1)), "a stage fits");
+  static_assert(AI == 2 * RB || (RB == 1 && AI == 1), "AI: activation DMAs per stage, 8 rows each");
   __shared__ __attribute__((aligned(16))) uint8_t lds[T::bytes];
   typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
@@ -108,11 +106,10 @@ __global__ __launch_bounds__(64 * kDmWaves) void marlin_dense_mid_kernel(const v
   // grouped scales of the tile's columns, 8 pieces per chunk
   const char* gS =
       reinterpret_cast<const char*>(a.s) + ((size_t)(q0 >> 1) * (uint32_t)N + n0) * 2 + 16 * cmin(lane, 8 * NCH - 1);
-  uint8_t* const wlds = lds + wave * (D * T::stage_b);  // this wave's ring
-  const uint32_t wlds_addr = (uint32_t)(size_t)(lds_u8*)lds + (uint32_t)(wave * (D * T::stage_b));
-  // DMAs of this wave's next stage into its buffer b (uniform)
-  auto issue = [&](int b) {
-    const uint32_t lb = wlds_addr + (uint32_t)(b * T::stage_b);
+  uint8_t* const wlds = lds + wave * T::stage_b;  // this wave's buffer
+  const uint32_t lb = (uint32_t)(size_t)(lds_u8*)lds + (uint32_t)(wave * T::stage_b);
+  // DMAs of this wave's next stage
+  auto issue = [&] {
 #pragma unroll
     for (int u = 0; u < 2 * NCH; u++)
       dma16x1(lb + WOFF + 1024 * u, wv + (uint32_t)(u & 1) * 2 * rowB + 512 * (u >> 1), gB);
@@ -126,10 +123,7 @@ __global__ __launch_bounds__(64 * kDmWaves) void marlin_dense_mid_kernel(const v
     gB += (size_t)(KG * 4) * rowB;
   };
 
-  // prologue: the first D stages
-#pragma unroll
-  for (int i = 0; i < D; i++)
-    if (i < mine) issue(i);
+  if (mine > 0) issue();  // uniform
 
   // ---- MFMA lane roles.  The weight is the A operand of v_mfma_f32_16x16x32_f16 (rows =
   // output columns), the activations the B operand.  Lane (rho, h) holds column
@@ -170,7 +164,7 @@ __global__ __launch_bounds__(64 * kDmWaves) void marlin_dense_mid_kernel(const v
       act[rb][0] = *reinterpret_cast<const half8_t*>(st + o_act0 + 2048 * rb);
       act[rb][1] = *reinterpret_cast<const half8_t*>(st + o_act1 + 2048 * rb);
     }
-    // the stage is in registers: its buffer is free for the stage D later
+    // the stage is in registers: its buffer is free for the next one
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     refill();
     __builtin_amdgcn_sched_barrier(0);
@@ -208,17 +202,14 @@ __global__ __launch_bounds__(64 * kDmWaves) void marlin_dense_mid_kernel(const v
     }
   };
 
-  // ---- main loop: a wave waits for its own DMAs of stage s (at most D - 1 later stages
-  // are in flight), reads the stage into registers, refills its buffer, computes ----
-  int buf = 0;
+  // ---- main loop: a wave waits for its own DMAs of stage s, reads the stage into
+  // registers, sends for the next one and computes ----
   for (int s = 0; s < mine; s++) {
-    if (s + D <= mine) wait_vm<L * (D - 1)>();
-    else wait_stages<L, cmax(1, D - 1)>(mine - 1 - s);
-    compute(wlds + buf * T::stage_b, [&] {
-      if (s + D < mine) issue(buf);
+    wait_vm<0>();
+    compute(wlds, [&] {
+      if (s + 1 < mine) issue();
     });
     __builtin_amdgcn_sched_barrier(0);
-    buf = buf + 1 == D ? 0 : buf + 1;
   }
 
   // ---- reduction: the 8 waves' sums, RC 16-row blocks at a time, in wave order; thread

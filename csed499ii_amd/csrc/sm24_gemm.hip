@@ -871,14 +871,14 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
 }
 
 // Tile and K splits of the mid-batch kernel (33-192 rows), from a cost model fitted to
-// 1000 forced plans (every tile x splits 1-8 on ten K x N, 2048x2048 to 28672x8192, M in
-// {33, 48, 64, 80, 96, 131, 160, 192}, one box; mean error 4 %, the model's choices 1 %
-// from the best of each call): a fixed cost, the stages of a wave at the tile's measured
-// stage time, the reduction in LDS (by tile size), and for a split the exchange of the
-// fp32 partials.  Only plans of one workgroup per CU in one round are considered: a
-// second round loses to the large-M kernel (7B gate_up at M = 96 31.1 against 24.2 us,
-// 4096x12288 at M = 131 24.9 against 21.4), as does K above 16384 beyond 64 rows
-// (28672x8192 at M = 96: 49.9 against 46.3).  splits == 0: no such plan.
+// 3000 forced plans (every tile x splits 1-8 on sixteen K x N, 1024x1024 to 8192x57344, M
+// from 12 to 1024, one box; mean error 6 %, the model's choices 1.4 % from the best of
+// each call): a fixed cost, the stages of a wave at the tile's measured stage time, the
+// reduction in LDS (by tile size), and for a split the exchange of the fp32 partials.
+// Only plans of one workgroup per CU in one round are considered (splits == 0: none): a
+// second round loses to the large-M kernel (7B gate_up at M = 96 28.1 against 23.7 us,
+// 4096x12288 at M = 192 26.9 against 22.7), as does K above 16384 beyond 64 rows
+// (28672x8192 at M = 160: 74.3 against 70.3).
 // MARLIN_HIP_MID=0 turns the kernel off (read once).
 constexpr int kMidMaxM = 192;
 MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
@@ -887,25 +887,24 @@ MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
     int ncb, rb;
     double stage_us;
   };
-  static const Cand cands[] = {{4, 1, 0.45}, {4, 2, 0.54}, {4, 3, 0.72}, {4, 4, 0.82},
-                               {4, 5, 0.95}, {8, 2, 0.87}, {8, 3, 1.07}, {8, 4, 1.10}};
+  static const Cand cands[] = {{4, 1, 0.52}, {4, 2, 0.63}, {4, 3, 0.74}, {4, 4, 0.88}, {4, 5, 1.05},
+                               {8, 2, 0.90}, {8, 3, 1.02}, {8, 4, 1.15}};
   MidShape best{0, 0, 0};
-  if (!on || M <= kDecodeMaxM || M > kMidMaxM || K % 64 != 0 || (K > 16384 && M > 64) ||
-      (long long)M * K >= (1LL << 31))
+  if (!on || M <= kDecodeMaxM || M > kMidMaxM || K % 64 != 0 || (K > 16384 && M > 64) || (long long)M * K >= (1LL << 31))
     return best;
-  // Narrow N at up to 64 rows, K from 4096: the launches a query of the plan expects
-  // there are two, so K is split and a second launch adds the partials (4096x4096 at
-  // M = 64: one unsplit launch of 16-row tiles takes 8.0 us).
+  // Narrow N at 33-64 rows, K from 4096: the launches a query of the plan expects there are
+  // two, so K is split and a second launch adds the partials (4096x4096 at M = 64: one
+  // unsplit launch of 16-row tiles takes 6.9 us).
   const bool two = !nosplit && M <= kDecodeMidMaxM && 2 * (N / 64) < cus && K >= 4096;
   double best_cost = 1e30;
   for (const Cand& c : cands) {
     if (N % (16 * c.ncb) != 0) continue;
-    const int tiles = N / (16 * c.ncb) * ((M + 16 * c.rb - 1) / (16 * c.rb));
+    const long long tiles = (long long)(N / (16 * c.ncb)) * ((M + 16 * c.rb - 1) / (16 * c.rb));
     for (int s = two ? 2 : 1; s <= (nosplit ? 1 : 8) && tiles * s <= cus; s++) {
       if (s > 1 && K / 64 < 8 * s) break;
       const double x = (double)(tiles * s) / cus;
-      double cost = 3.1 + ((K / 64 + s - 1) / s + 7) / 8 * c.stage_us * (1 + 0.18 * (x - 0.75)) + 0.096 * c.ncb * c.rb;
-      if (s > 1) cost += 1.1 + 8.0 * s * M * (double)N / 5.3e6;
+      double cost = 2.3 + (K / 64 / s + 7) / 8 * c.stage_us * (1 + 0.29 * (x - 0.75)) + 0.118 * c.ncb * c.rb;
+      if (s > 1) cost += 1.13 + 8.0 * s * M * (double)N / 4.9e6;
       if (cost < best_cost) {
         best_cost = cost;
         best = MidShape{c.ncb, c.rb, s, two};
@@ -946,8 +945,8 @@ int validate(int prob_m, int prob_n, int prob_k, int groupsize, int thread_k, in
 enum : int { KERNEL_DECODE = 0, KERNEL_PREFILL = 1, KERNEL_GENERAL = 2, KERNEL_DECODE_DMA = 3, KERNEL_MID = 4 };
 
 // The kernel a call on the reference layout runs (after 3-bit operands at large M are
-// expanded to 4 bits): the mid-batch kernel at 33-192 rows where it covers the call in
-// one round, else the decode kernel up to 32 rows, and below the large-M
+// expanded to 4 bits): the mid-batch kernel at 33-192 rows where it covers the call
+// in one round, else the decode kernel up to 32 rows, and below the large-M
 // kernel's threshold up to 96 rows as consecutive launches of <= 32 rows (measured
 // on the Llama-2-7B shapes: o at M = 64 17.8 against 28.8 us, down at M = 96 40.5
 // against 49.7 us for the general kernel); the large-M kernel where it fits; the

@@ -13,15 +13,18 @@
 // path from L2 into a compute unit moves 64 bytes per clock.  So they come by LDS-DMA in
 // whole 128-byte lines, 8 rows to an instruction (every CU reading the same 64 rows of
 // K = 4096: 5.8 us with the launch, against 7.2 in 64-byte pieces and 17 by loads into
-// registers in operand order), into a ring that takes the whole LDS.  A wave reads a due
-// stage into registers in one go and refills its buffer before it computes, so D stages
-// per wave stay in flight.  At 64 rows of 7B qkv the LDS is busy 29 % of the cycles, the
-// matrix cores 19 % and the VALU 25 %: latency, with two waves per SIMD, is what is left.
+// registers in operand order).  A wave has one stage buffer: it reads the due stage into
+// registers in one go, sends for the next one into the same buffer and computes meanwhile.
+// More stages in flight were slower on every call (buffers for 1 / 2 / 4 stages, us: 7B
+// qkv at M = 64 12.3 / 13.8 / 13.8, o at M = 131 8.6 / 9.6 / 9.8, 70B o at M = 64 15.3 /
+// 15.9 / 16.8): a wave's DMAs return in order, so the first stage waits for less, and the
+// smaller LDS lets two workgroups share a compute unit.  4, 12 and 16 waves were slower
+// than 8.
 //
-// Against two decode launches of 32 rows, or the large-M kernel, us per call on one box:
-// M = 64 7B qkv 18.9 -> 14.1, gate_up 21.3 -> 19.1, down 20.2 -> 13.7, 70B o 24.3 ->
-// 16.3, down 56.7 -> 39.3; M = 131 7B o 15.9 -> 9.8, down 23.1 -> 20.1, 70B qkv 35.9 ->
-// 26.9; 2048x2048 at M = 96 17.4 -> 5.6, 1024x5120 at M = 48 11.8 -> 4.5.
+// us per call on one box, against the decode launches of up to 32 rows or the large-M
+// kernel: M = 64 7B qkv 18.9 -> 12.4, o 14.6 -> 8.4 (two launches), gate_up 21.3 -> 19.0,
+// down 20.2 -> 12.5, 70B o 24.3 -> 15.2, down 56.7 -> 33.7; M = 131 7B o 15.9 -> 8.6, 70B
+// qkv 35.9 -> 24.0; 2048x2048 at M = 96 17.4 -> 5.2.
 #pragma once
 #include "sm24_decode_dma.h"
 #include "sm24_host.h"
@@ -30,7 +33,7 @@ namespace sm24 {
 
 constexpr int kMidWaves = 8;
 
-// One wave's ring: D stages of its own activation rows and weight side; the
+// One wave's stage buffer (its activation rows and weight side of one k-pair); the
 // workgroup's reduction buffer lies in the same space.
 template <int NCB, int RB, bool GROUPED, int VF, int MF>
 struct MidLds {
@@ -41,13 +44,13 @@ struct MidLds {
   static constexpr int sc_n = GROUPED ? TC / 8 : 0;
   static constexpr int nms = 2 * mpk + sc_n;                   // metadata and scale pieces of a stage
   static constexpr int stage_b = act_b + 16 * (2 * bpk + nms);
-  static constexpr int vdma = (2 * bpk + 63) / 64, msdma = (nms + 63) / 64;
-  static constexpr int L = 2 * RB + vdma + msdma;              // DMA instructions per stage
-  static constexpr int D = cmin(4, cmin(160 * 1024 / (kMidWaves * stage_b), 60 / L + 1));
+  static constexpr int vdma = (2 * bpk + 63) / 64, msdma = (nms + 63) / 64;  // weight DMAs
   static constexpr int redp = TC + 4;                          // floats of one reduction row
   static constexpr int red_row = kMidWaves * 16 * redp * 4;    // 16 rows of every wave
-  static constexpr int RC = cmin(RB, 160 * 1024 / red_row);    // 16-row blocks reduced at a time
-  static constexpr int bytes = cmax(D * kMidWaves * stage_b, RC * red_row);
+  // 16-row blocks reduced at a time: half the LDS where the registers let two workgroups
+  // share a compute unit
+  static constexpr int RC = cmin(RB, (NCB * RB <= 12 ? 80 : 160) * 1024 / red_row);
+  static constexpr int bytes = cmax(kMidWaves * stage_b, RC * red_row);
 };
 
 template <int NCB, int RB, bool GROUPED, int VF, int MF>
@@ -56,10 +59,10 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
                                                                   int K_, int splits_, GemmArgs a_) {
   const GemmArgs a = with_lead(a_, B_, meta_, s_, A_, zeros_, M_, N_, K_, splits_);
   using T = MidLds<NCB, RB, GROUPED, VF, MF>;
-  constexpr int D = T::D, L = T::L, MB = 16 * RB, TC = T::TC, KG = kMidWaves;
+  constexpr int MB = 16 * RB, TC = T::TC, KG = kMidWaves;
   constexpr int BPK = T::bpk, MPK = T::mpk, NMS = T::nms;
   constexpr int VOFF = T::act_b, MOFF = VOFF + 32 * BPK, SOFF = MOFF + 32 * MPK;
-  static_assert(D >= 1 && BPK <= 64, "a stage fits; one k-block of values per instruction");
+  static_assert(T::bytes <= 160 * 1024 && BPK <= 64, "one k-block of values per instruction");
   __shared__ __attribute__((aligned(16))) uint8_t lds[T::bytes];
   typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
@@ -130,11 +133,10 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
       ms_inc[u] = KG / 2 * 2 * (uint32_t)N;
     }
   }
-  uint8_t* const wlds = lds + wave * (D * T::stage_b);  // this wave's ring
-  const uint32_t wlds_addr = (uint32_t)(size_t)(lds_u8*)lds + (uint32_t)(wave * (D * T::stage_b));
-  // DMAs of this wave's next stage into its buffer b (uniform)
-  auto issue = [&](int b) {
-    const uint32_t lb = wlds_addr + (uint32_t)(b * T::stage_b);
+  uint8_t* const wlds = lds + wave * T::stage_b;  // this wave's buffer
+  const uint32_t lb = (uint32_t)(size_t)(lds_u8*)lds + (uint32_t)(wave * T::stage_b);
+  // DMAs of this wave's next stage
+  auto issue = [&] {
     static_for<0, T::vdma>([&](auto ui) {
       constexpr int u = decltype(ui)::value;
       if constexpr (VN == 64) dma16x1(lb + VOFF + 16 * VN * u, val_v[u], gB);
@@ -151,10 +153,7 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
     gB += (size_t)(KG * 2 * bpc) * (uint32_t)N;
   };
 
-  // prologue: the first D stages
-#pragma unroll
-  for (int i = 0; i < D; i++)
-    if (i < mine) issue(i);
+  if (mine > 0) issue();  // uniform
 
   // ---- MFMA lane roles (as in sm24_decode_kernel) ----
   const int h = lane >> 4, rho = lane & 15;
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
           act[rb] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
         }
       }
-      // the stage is in registers: its buffer is free for the stage D later
+      // the stage is in registers: its buffer is free for the next one
       if (c0 + HB == NCB) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         refill();
@@ -301,17 +300,14 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
     }
   };
 
-  // ---- main loop: a wave waits for its own DMAs of stage s (at most D - 1 later stages
-  // are in flight), reads the stage into registers, refills its buffer, computes ----
-  int buf = 0;
+  // ---- main loop: a wave waits for its own DMAs of stage s, reads the stage into
+  // registers, sends for the next one and computes ----
   for (int s = 0; s < mine; s++) {
-    if (s + D <= mine) wait_vm<L * (D - 1)>();
-    else wait_stages<L, cmax(1, D - 1)>(mine - 1 - s);
-    compute(wlds + buf * T::stage_b, [&] {
-      if (s + D < mine) issue(buf);
+    wait_vm<0>();
+    compute(wlds, [&] {
+      if (s + 1 < mine) issue();
     });
     __builtin_amdgcn_sched_barrier(0);
-    buf = buf + 1 == D ? 0 : buf + 1;
   }
 
   // ---- reduction: the 8 waves' sums, RC 16-row blocks at a time, in wave order; thread
