@@ -48,6 +48,8 @@ _lib: ctypes.CDLL | None = None
 def load() -> ctypes.CDLL:
     """Load the library once and set the argument types of every export."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not LIB_PATH.exists():

@@ -61,6 +61,12 @@ def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
 
 
+#: HIP stream handle that torch's current stream of device ``index`` stands for, without
+#: the Stream object that ``torch.cuda.current_stream`` makes on each call.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _check_operands(A, B, meta, C, s, workspace, b_elems: int, b_dtype: torch.dtype, meta_elems: int,
                     meta_dtype: torch.dtype):
     """Device, dtype, contiguity and size checks (``meta`` and ``workspace`` may be
@@ -102,6 +108,47 @@ def _check_operands(A, B, meta, C, s, workspace, b_elems: int, b_dtype: torch.dt
             raise RuntimeError(f"{name} must be 16-byte aligned")
 
 
+def _operands_fit(A, B, meta, C, s, workspace, M, N, b_elems: int, b_dtype: torch.dtype, meta_elems: int,
+                  meta_dtype: torch.dtype):
+    """The operands' addresses where everything that :func:`_check_operands` looks at
+    holds, else None: then that one names the fault (``meta_dtype`` None: the dense op,
+    which has no metadata).  An eager call of a few rows is bound by this host path, not
+    by its kernel of about 4 us, so each property is read once, in one pass."""
+    T, half = torch.Tensor, torch.half
+    if not (isinstance(A, T) and isinstance(B, T) and isinstance(C, T) and isinstance(s, T)
+            and isinstance(workspace, T) and (isinstance(meta, T) if meta_dtype is not None else meta is None)):
+        return None
+    dev = A.get_device()
+    if not (A.is_cuda and B.is_cuda and C.is_cuda and s.is_cuda and workspace.is_cuda
+            and B.get_device() == dev and C.get_device() == dev and s.get_device() == dev
+            and workspace.get_device() == dev
+            and A.is_contiguous() and B.is_contiguous() and C.is_contiguous() and s.is_contiguous()
+            and workspace.is_contiguous()
+            and A.dtype == half and C.dtype == half and s.dtype == half and B.dtype == b_dtype
+            and A.dim() == 2 and C.dim() == 2 and s.dim() == 2
+            and C.size(0) == M and s.size(1) == N and B.numel() == b_elems):
+        return None
+    a, b, c, sp, w = A.data_ptr(), B.data_ptr(), C.data_ptr(), s.data_ptr(), workspace.data_ptr()
+    if meta_dtype is None:
+        m = 0
+    elif (meta.is_cuda and meta.get_device() == dev and meta.is_contiguous() and meta.dtype == meta_dtype
+          and meta.numel() == meta_elems):
+        m = meta.data_ptr()
+    else:
+        return None
+    return None if (a | b | c | sp | w | m) & 15 else (a, b, m, c, sp, w, dev)
+
+
+def _operands(A, B, meta, C, s, workspace, M, N, b_elems, b_dtype, meta_elems, meta_dtype):
+    """Checked operands: ``(A, B, meta, C, s, workspace)`` addresses, device index."""
+    fit = _operands_fit(A, B, meta, C, s, workspace, M, N, b_elems, b_dtype, meta_elems, meta_dtype)
+    if fit is None:
+        _check_operands(A, B, meta, C, s, workspace, b_elems, b_dtype, meta_elems, meta_dtype)
+        fit = (A.data_ptr(), B.data_ptr(), 0 if meta_dtype is None else meta.data_ptr(), C.data_ptr(), s.data_ptr(),
+               workspace.data_ptr(), A.get_device())
+    return fit
+
+
 def _groupsize_and_checks(A, C, s, workspace, max_par):
     """Shape inference and checks of the reference binding (marlin_cuda.cpp:66-80)."""
     prob_n = A.size(0)
@@ -132,14 +179,12 @@ def _call(fn_name, A, B, meta, C, s, workspace, thread_k, thread_m, sms, max_par
           meta_elems_fn, meta_dtype):
     lib = _lib.load()
     prob_m, prob_n, prob_k, groupsize = _groupsize_and_checks(A, C, s, workspace, max_par)
-    _check_operands(A, B, meta, C, s, workspace, b_elems_fn(prob_k, prob_m), b_dtype,
-                    meta_elems_fn(prob_k, prob_m), meta_dtype)
-    dev = A.get_device()
-    stream = torch.cuda.current_stream(A.device).cuda_stream
-    err = getattr(lib, fn_name)(_ptr(A), _ptr(B), _ptr(meta), _ptr(C), _ptr(s), prob_m, prob_n, prob_k,
-                                _ptr(workspace), groupsize, dev, ctypes.c_void_p(stream), thread_k, thread_m,
-                                sms, max_par)
-    _raise_for(err, prob_m, prob_n, prob_k, thread_k, thread_m, groupsize)
+    a, b, m, c, sp, w, dev = _operands(A, B, meta, C, s, workspace, prob_n, prob_m,
+                                       b_elems_fn(prob_k, prob_m), b_dtype, meta_elems_fn(prob_k, prob_m), meta_dtype)
+    err = getattr(lib, fn_name)(a, b, m, c, sp, prob_m, prob_n, prob_k, w, groupsize, dev, _raw_stream(dev), thread_k,
+                                thread_m, sms, max_par)
+    if err:
+        _raise_for(err, prob_m, prob_n, prob_k, thread_k, thread_m, groupsize)
 
 
 def mul_2_4(A, B, meta, C, s, workspace, thread_k=-1, thread_m=-1, sms=-1, max_par=16):
@@ -177,10 +222,10 @@ def mul(A, B, C, s, workspace, thread_k=-1, thread_n=-1, sms=-1, max_par=16):
         raise RuntimeError(f"k={prob_k} not compatible with {s.size(0)} groups.")
     if workspace.numel() < prob_n // 128 * max_par:
         raise RuntimeError(f"workspace must be of size at least {prob_n // 128 * max_par}.")
-    _check_operands(A, B, None, C, s, workspace, prob_k * prob_n // 8, torch.int32, 0, torch.int16)
-    stream = torch.cuda.current_stream(A.device).cuda_stream
-    err = lib.marlin_hip_mul(_ptr(A), _ptr(B), _ptr(C), _ptr(s), prob_m, prob_n, prob_k, _ptr(workspace),
-                             groupsize, A.get_device(), ctypes.c_void_p(stream), thread_k, thread_n, sms, max_par)
+    a, b, _, c, sp, w, dev = _operands(A, B, None, C, s, workspace, prob_m, prob_n, prob_k * prob_n // 8,
+                                       torch.int32, 0, None)
+    err = lib.marlin_hip_mul(a, b, c, sp, prob_m, prob_n, prob_k, w, groupsize, dev, _raw_stream(dev), thread_k,
+                             thread_n, sms, max_par)
     if err == _lib.OK:
         return
     if err == _lib.ERR_PROB_SHAPE:
@@ -571,15 +616,18 @@ class Layer_2_4(nn.Module):
             module.to_native()
 
     def forward(self, A):
-        C = torch.empty(A.shape[:-1] + (self.s.shape[1],), dtype=A.dtype, device=A.device)
-        A2, C2 = A.view((-1, A.shape[-1])), C.view((-1, C.shape[-1]))
-        if getattr(self, "Bn", None) is not None and A2.shape[0] <= self.NATIVE_MAX_ROWS and self.Bn.device == A.device:
-            mul_2_4_native(A2, self.Bn, self.metan, C2, self.sn)
-            return C
+        s, device = self.s, A.device
+        C = torch.empty(A.shape[:-1] + (s.shape[1],), dtype=A.dtype, device=device)
+        A2, C2 = (A, C) if A.dim() == 2 else (A.view((-1, A.shape[-1])), C.view((-1, C.shape[-1])))
+        # (a failed attribute lookup on a module costs an exception)
+        if "Bn" in self._buffers or "Bn" in self.__dict__:
+            if self.Bn is not None and A2.shape[0] <= self.NATIVE_MAX_ROWS and self.Bn.device == device:
+                mul_2_4_native(A2, self.Bn, self.metan, C2, self.sn)
+                return C
         ws = self.workspace
-        if ws.device != A.device:
-            ws = self.workspace = ws.to(A.device)
-        mul_2_4(A2, self.B, self.meta, C2, self.s, ws)
+        if ws.device != device:
+            ws = self.workspace = ws.to(device)
+        mul_2_4(A2, self.B, self.meta, C2, s, ws)
         return C
 
     #: Largest batch that ``forward`` runs on the lane-native copy made by
@@ -700,11 +748,13 @@ class Layer(nn.Module):
         self.register_buffer("workspace", torch.zeros(self.n // 128 * 16, dtype=torch.int), persistent=False)
 
     def forward(self, A):
-        C = torch.empty(A.shape[:-1] + (self.s.shape[1],), dtype=A.dtype, device=A.device)
+        s, device = self.s, A.device
+        C = torch.empty(A.shape[:-1] + (s.shape[1],), dtype=A.dtype, device=device)
         ws = self.workspace
-        if ws.device != A.device:
-            ws = self.workspace = ws.to(A.device)
-        mul(A.view((-1, A.shape[-1])), self.B, C.view((-1, C.shape[-1])), self.s, ws)
+        if ws.device != device:
+            ws = self.workspace = ws.to(device)
+        A2, C2 = (A, C) if A.dim() == 2 else (A.view((-1, A.shape[-1])), C.view((-1, C.shape[-1])))
+        mul(A2, self.B, C2, s, ws)
         return C
 
     def pack(self, linear, scales, trans=False):

@@ -542,3 +542,48 @@ def test_per_column_scales_full_size(M, K, N):
     for c0 in (0, chunks // 2 - 2, chunks - 4):
         ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
         assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"g=-1 {K}x{N} M={M} slice {c0}")
+
+
+def _bad_operands():
+    """One fault per entry: which operand, and what replaces it."""
+    yield "A", lambda t: t.float()
+    yield "A", lambda t: t.t().contiguous().t()
+    yield "A", lambda t: t.cpu()
+    yield "A", lambda t: t.view(1, *t.shape)
+    yield "A", lambda t: torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    yield "B", lambda t: t[:-1]
+    yield "B", lambda t: t.view(torch.int16)
+    yield "B", lambda t: t.cpu()
+    yield "meta", lambda t: t.view(torch.int32)
+    yield "meta", lambda t: t[:-1]
+    yield "meta", lambda t: None
+    yield "meta", lambda t: t.cpu()
+    yield "C", lambda t: t[:-1]
+    yield "C", lambda t: t.bfloat16()
+    yield "s", lambda t: t[:, :-16].contiguous()
+    yield "s", lambda t: t[0]
+    yield "s", lambda t: t.cpu()
+    yield "workspace", lambda t: t.cpu()
+    yield "workspace", lambda t: None
+    yield "workspace", lambda t: t.view(-1, 1).expand(-1, 2)
+
+
+@pytest.mark.parametrize("i", range(len(list(_bad_operands()))))
+def test_refused_operands(i):
+    """The one-pass operand test lets through nothing that the checks refuse, and the
+    error is the checks' own."""
+    M, K, N = 4, 256, 256
+    wt = synth.make_weight(K, N, synth.SEED_BASE, 128, device=DEV)
+    ops = {"A": torch.ones((M, K), dtype=torch.half, device=DEV), "B": wt["B"], "meta": wt["meta"],
+           "C": torch.zeros((M, N), dtype=torch.half, device=DEV), "s": wt["s"],
+           "workspace": torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)}
+    marlin.mul_2_4(**ops)
+    C = ops["C"].clone()
+    ops["C"].zero_()
+    name, fault = list(_bad_operands())[i]
+    bad = dict(ops, **{name: fault(ops[name])})
+    with pytest.raises((TypeError, RuntimeError, AttributeError, IndexError)):
+        marlin.mul_2_4(**bad)
+    assert not ops["C"].any()
+    marlin.mul_2_4(**ops)
+    assert torch.equal(ops["C"], C)
