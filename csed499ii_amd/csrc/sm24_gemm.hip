@@ -870,7 +870,7 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
          (long long)M * K < (1LL << 31) - 2048 && (long long)K * N < (1LL << 34);
 }
 
-// Tile and K splits of the mid-batch kernel (33-192 rows), from a cost model fitted to
+// Tile and K splits of the mid-batch kernel (17-192 rows), from a cost model fitted to
 // 3000 forced plans (every tile x splits 1-8 on sixteen K x N, 1024x1024 to 8192x57344, M
 // from 12 to 1024, one box; mean error 6 %, the model's choices 1.4 % from the best of
 // each call): a fixed cost, the stages of a wave at the tile's measured stage time, the
@@ -879,8 +879,17 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
 // second round loses to the large-M kernel (7B gate_up at M = 96 28.1 against 23.7 us,
 // 4096x12288 at M = 192 26.9 against 22.7), as does K above 16384 beyond 64 rows
 // (28672x8192 at M = 160: 74.3 against 70.3).
+// From 17 rows on: there it replaces the 32-row decode launches and their K splits (us per
+// call at M = 17 / 24 / 32, weights cold, one box, decode -> this kernel: 7B qkv 10.4 /
+// 10.3 / 10.3 -> 9.5 / 9.6 / 9.8, o 7.4 / 7.4 / 7.5 -> 6.9 / 6.9 / 6.6, down 10.2 / 10.2 /
+// 10.4 -> 9.5 / 9.4 / 9.7, 70B qkv 15.3 / 16.2 / 17.4 -> 13.1 / 13.5 / 14.0, o 12.0 / 12.9 /
+// 13.6 -> 11.8 / 12.0 / 12.4, down 28.6 / 31.7 / 34.1 -> 24.7 / 25.0 / 25.7, 2048x2048 5.8 /
+// 5.9 / 6.0 -> 4.5), but not at 12 rows, where those stage 16 (7B qkv 8.1 against 9.1,
+// 2048x2048 3.6 against 4.5).  Where the 64-column tiles pass one round of the CUs, the
+// decode launches up to 32 rows keep their split tail, which callers that query the plan
+// expect (4096x22016 at M = 17 / 24 13.6 / 14.7 against 13.8 / 14.1).
 // MARLIN_HIP_MID=0 turns the kernel off (read once).
-constexpr int kMidMaxM = 192;
+constexpr int kMidMinM = 17, kMidMaxM = 192;
 MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
   static const int on = env_choice("MARLIN_HIP_MID", {0, 1}, 1);
   struct Cand {
@@ -890,12 +899,12 @@ MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
   static const Cand cands[] = {{4, 1, 0.52}, {4, 2, 0.63}, {4, 3, 0.74}, {4, 4, 0.88}, {4, 5, 1.05},
                                {8, 2, 0.90}, {8, 3, 1.02}, {8, 4, 1.15}};
   MidShape best{0, 0, 0};
-  if (!on || M <= kDecodeMaxM || M > kMidMaxM || K % 64 != 0 || (K > 16384 && M > 64) || (long long)M * K >= (1LL << 31))
-    return best;
+  if (!on || M < kMidMinM || M > kMidMaxM || K % 64 != 0 || (long long)M * K >= (1LL << 31)) return best;
+  if ((M <= kDecodeMaxM && N / 64 > cus) || (K > 16384 && M > 64)) return best;
   // Narrow N at 33-64 rows, K from 4096: the launches a query of the plan expects there are
   // two, so K is split and a second launch adds the partials (4096x4096 at M = 64: one
   // unsplit launch of 16-row tiles takes 6.9 us).
-  const bool two = !nosplit && M <= kDecodeMidMaxM && 2 * (N / 64) < cus && K >= 4096;
+  const bool two = !nosplit && M > kDecodeMaxM && M <= kDecodeMidMaxM && 2 * (N / 64) < cus && K >= 4096;
   double best_cost = 1e30;
   for (const Cand& c : cands) {
     if (N % (16 * c.ncb) != 0) continue;
@@ -945,7 +954,7 @@ int validate(int prob_m, int prob_n, int prob_k, int groupsize, int thread_k, in
 enum : int { KERNEL_DECODE = 0, KERNEL_PREFILL = 1, KERNEL_GENERAL = 2, KERNEL_DECODE_DMA = 3, KERNEL_MID = 4 };
 
 // The kernel a call on the reference layout runs (after 3-bit operands at large M are
-// expanded to 4 bits): the mid-batch kernel at 33-192 rows where it covers the call
+// expanded to 4 bits): the mid-batch kernel at 17-192 rows where it covers the call
 // in one round, else the decode kernel up to 32 rows, and below the large-M
 // kernel's threshold up to 96 rows as consecutive launches of <= 32 rows (measured
 // on the Llama-2-7B shapes: o at M = 64 17.8 against 28.8 us, down at M = 96 40.5

@@ -1,4 +1,4 @@
-// Mid-sized batches (33 to 192 rows) of the 2:4 INT4 x FP16 GEMM for gfx950, where one
+// Mid-sized batches (17 to 192 rows) of the 2:4 INT4 x FP16 GEMM for gfx950, where one
 // workgroup per tile and K split covers the call in one round over the compute units.
 //
 // Work decomposition: a workgroup of 8 waves owns a tile of 16 NCB output columns (64 or

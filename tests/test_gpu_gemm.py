@@ -225,6 +225,33 @@ def test_mid_batches(M, N, K, g):
         assert torch.equal(_run(wt, A), C), "repeated calls differ"
 
 
+@pytest.mark.parametrize("M,N,K,g", [(17, 256, 64, -1), (17, 16384, 1024, -1), (24, 8192, 28672, 128),
+                                     (31, 10240, 832, -1), (32, 2048, 2176, 128), (20, 4096, 4096, 128)])
+def test_mid_batches_from_17_rows(M, N, K, g):
+    """The mid-batch kernel at 17-32 rows in one launch: one k-pair and odd counts of
+    them, one full round of 64-column tiles (N = 16384), K splits; column slices against
+    the oracle, nothing past C's end, the unsplit call of the no-allocation entry point
+    agrees, repeated calls bit-identical.  16 rows and wider N stay on the decode kernels."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    p = marlin.plan_2_4(M, K, N, g, sms=cus)
+    assert p["threads"] == 512 and p["kernel"] == "decode_dma" and p["launches"] == 1
+    wt, A = _problem(M, N, K, g, 8300 + M + K + N)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C, U = buf[:M * N].view(M, N), torch.empty((M, N), dtype=torch.half, device=DEV)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    marlin.mul_2_4(A, wt["B"], wt["meta"], C, wt["s"], ws)
+    marlin.mul_2_4_noalloc(A, wt["B"], wt["meta"], U, wt["s"])
+    torch.cuda.synchronize()
+    assert torch.isfinite(C).all() and bool((buf[M * N:] == 7.0).all())
+    t = to_cpu(wt)
+    for c0 in sorted({0, max(N // 128 - 2, 0), N // 64 - 4}):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        for X in (C, U):
+            assert_close(X[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"M={M} {K}x{N} g={g} slice {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
 @pytest.mark.parametrize("M,K,N", [(64, 4096, 4096), (131, 11008, 4096), (48, 8192, 10240)])
 def test_mid_graph_replay_and_noalloc(M, K, N):
     """Captured mid-batch calls that split K (a second launch, or the hand-off in the
