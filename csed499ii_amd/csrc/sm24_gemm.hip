@@ -870,7 +870,7 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
          (long long)M * K < (1LL << 31) - 2048 && (long long)K * N < (1LL << 34);
 }
 
-// Tile and K splits of the mid-batch kernel (17-192 rows), from a cost model fitted to
+// Tile and K splits of the mid-batch kernel (17-192 rows; narrow N up to 1024), from a cost model fitted to
 // 3000 forced plans (every tile x splits 1-8 on sixteen K x N, 1024x1024 to 8192x57344, M
 // from 12 to 1024, one box; mean error 6 %, the model's choices 1.4 % from the best of
 // each call): a fixed cost, the stages of a wave at the tile's measured stage time, the
@@ -890,6 +890,15 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
 // expect (4096x22016 at M = 17 / 24 13.6 / 14.7 against 13.8 / 14.1).
 // MARLIN_HIP_MID=0 turns the kernel off (read once).
 constexpr int kMidMinM = 17, kMidMaxM = 192;
+// Narrow N (below 4096) leaves the large-M kernel a few workgroups that split K up to eight
+// ways: there more rows are still one round of this kernel (us per call at M = 200 / 512 /
+// 1000, one box, large-M -> this kernel: 1024x1024 13.0 / 13.9 / 11.5 -> 3.9 / 4.2 / 5.7,
+// 2048x2048 16.8 / 17.7 / 17.7 -> 5.5 / 7.3 / 12.1, 4096x2816 at 200 / 512 20.1 / 22.2 ->
+// 9.4 / 15.7, 8192x2048 24.0 / 26.6 / 34.5 -> 11.7 / 19.1 / 30.5).  At longer K its row
+// tiles read the weight too often from some row count on (11008x1536 26.0 / 31.3 / 36.9 ->
+// 14.5 / 26.1 / 39.0; 16384x3072 with 3-bit metadata at 200 / 333 / 512 38.5 / 44.6 / 50.7
+// -> 29.9 / 44.8 / 52.0).
+int mid_max_m(int N, int K) { return N >= 4096 ? kMidMaxM : K <= 8192 ? 1024 : K <= 12288 ? 640 : 320; }
 MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
   static const int on = env_choice("MARLIN_HIP_MID", {0, 1}, 1);
   struct Cand {
@@ -899,7 +908,7 @@ MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
   static const Cand cands[] = {{4, 1, 0.52}, {4, 2, 0.63}, {4, 3, 0.74}, {4, 4, 0.88}, {4, 5, 1.05},
                                {8, 2, 0.90}, {8, 3, 1.02}, {8, 4, 1.15}};
   MidShape best{0, 0, 0};
-  if (!on || M < kMidMinM || M > kMidMaxM || K % 64 != 0 || (long long)M * K >= (1LL << 31)) return best;
+  if (!on || M < kMidMinM || M > mid_max_m(N, K) || K % 64 != 0 || (long long)M * K >= (1LL << 31)) return best;
   if ((M <= kDecodeMaxM && N / 64 > cus) || (K > 16384 && M > 64)) return best;
   // Narrow N at 33-64 rows, K from 4096: the launches a query of the plan expects there are
   // two, so K is split and a second launch adds the partials (4096x4096 at M = 64: one
@@ -954,8 +963,8 @@ int validate(int prob_m, int prob_n, int prob_k, int groupsize, int thread_k, in
 enum : int { KERNEL_DECODE = 0, KERNEL_PREFILL = 1, KERNEL_GENERAL = 2, KERNEL_DECODE_DMA = 3, KERNEL_MID = 4 };
 
 // The kernel a call on the reference layout runs (after 3-bit operands at large M are
-// expanded to 4 bits): the mid-batch kernel at 17-192 rows where it covers the call
-// in one round, else the decode kernel up to 32 rows, and below the large-M
+// expanded to 4 bits): the mid-batch kernel at 17-192 rows (narrow N: 1024) where it covers the
+// call in one round, else the decode kernel up to 32 rows, and below the large-M
 // kernel's threshold up to 96 rows as consecutive launches of <= 32 rows (measured
 // on the Llama-2-7B shapes: o at M = 64 17.8 against 28.8 us, down at M = 96 40.5
 // against 49.7 us for the general kernel); the large-M kernel where it fits; the
@@ -973,10 +982,13 @@ void describe(int M, int N, int K, int sms, bool noalloc, int out[5]) {
   const int kernel = kernel_for(M, N, K, sms, noalloc);
   out[0] = kernel;
   if (kernel == KERNEL_MID) {
-    // reported with the family of its batch: the large-M kernels from their threshold on,
-    // the LDS-DMA decode kernels below
+    // reported with the family of its batch: the large-M kernels from their threshold on
+    // (above 192 rows where they take the shape, else the multi-block one), the LDS-DMA
+    // decode kernels below
     const MidShape d = mid_plan(M, N, K, sms, noalloc);
-    out[0] = M >= prefill_min_m(N, K) ? KERNEL_PREFILL : KERNEL_DECODE_DMA;
+    out[0] = M > kMidMaxM && !prefill_fits(M, N, K, VAL4, META4) ? KERNEL_GENERAL
+             : M >= prefill_min_m(N, K)                         ? KERNEL_PREFILL
+                                                                : KERNEL_DECODE_DMA;
     out[1] = N / (16 * d.ncb) * ((M + 16 * d.rb - 1) / (16 * d.rb)) * d.splits;
     out[2] = 512;
     out[3] = d.splits;

@@ -252,6 +252,47 @@ def test_mid_batches_from_17_rows(M, N, K, g):
         assert torch.equal(_run(wt, A), C), "repeated calls differ"
 
 
+@pytest.mark.parametrize("M,N,K,g", [(193, 1024, 1024, 128), (200, 3840, 4096, 128), (300, 768, 2176, 128),
+                                     (513, 2048, 2048, -1), (640, 1536, 11008, 128), (1000, 1024, 8192, 128),
+                                     (1024, 1024, 64, -1), (333, 256, 8192, -1)])
+def test_mid_batches_narrow_n(M, N, K, g):
+    """The mid-batch kernel above 192 rows on narrow N: ragged row tiles, K splits and
+    none, one k-pair, widths of no other kernel but the multi-block one (768, 256); column
+    slices against the oracle, nothing past C's end, repeated calls bit-identical."""
+    p = marlin.plan_2_4(M, K, N, g)
+    assert p["threads"] == 512 and p["launches"] == 1
+    assert p["kernel"] == ("general" if N in (256, 768) or K == 64 else "large_m")
+    wt, A = _problem(M, N, K, g, 8500 + M + K + N)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C = buf[:M * N].view(M, N)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    marlin.mul_2_4(A, wt["B"], wt["meta"], C, wt["s"], ws)
+    torch.cuda.synchronize()
+    assert torch.isfinite(C).all() and bool((buf[M * N:] == 7.0).all())
+    t = to_cpu(wt)
+    for c0 in sorted({0, N // 64 - 4}):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"M={M} {K}x{N} g={g} slice {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
+@pytest.mark.parametrize("M,N,K,g", [(256, 4096, 128, 128), (300, 4096, 256, -1), (320, 4608, 384, 128),
+                                     (640, 8192, 1024, 128), (300, 4352, 8192, -1), (1100, 2048, 8192, 128)])
+def test_prefill_beyond_mid(M, N, K, g):
+    """The large-M kernel where the mid-batch one does not apply (N from 4096, or more
+    than 1024 rows): one to six scale groups' worth of k-steps, ragged row and column
+    tiles, K splits of few tiles; column slices, repeats bit-identical."""
+    assert marlin.plan_2_4(M, K, N, g)["kernel"] == "large_m"
+    wt, A = _problem(M, N, K, g, 8700 + M + K + N)
+    C = _run(wt, A)
+    t = to_cpu(wt)
+    for c0 in (0, N // 64 - 4):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"M={M} {K}x{N} g={g} slice {c0}")
+    assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
 @pytest.mark.parametrize("M,K,N", [(64, 4096, 4096), (131, 11008, 4096), (48, 8192, 10240)])
 def test_mid_graph_replay_and_noalloc(M, K, N):
     """Captured mid-batch calls that split K (a second launch, or the hand-off in the

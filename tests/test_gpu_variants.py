@@ -133,12 +133,12 @@ def test_w3_gemm_bit_exact_against_4bit_path(M, K, N):
 
 
 MID_CASES = [(64, 4096, 22016), (48, 4096, 4096), (131, 4096, 4096), (96, 2048, 10240), (80, 1024, 12288),
-             (40, 8192, 10240)]
+             (40, 8192, 10240), (24, 8192, 8192), (513, 2048, 2048), (300, 4096, 768)]
 
 
 @pytest.mark.parametrize("M,K,N", MID_CASES)
 def test_mid_batches_3bit(M, K, N):
-    """The mid-batch kernel (33-192 rows) on 3-bit metadata and 3-bit values: the same
+    """The mid-batch kernel (17-192 rows, narrow N up to 1024) on 3-bit metadata and 3-bit values: the same
     tiles and order of sums as 4-bit operands, so bit-identical to the 4-bit calls."""
     assert marlin.plan_2_4(M, K, N)["threads"] == 512
     A = synth.make_activation(M, K, 7 + M, device=DEV)
