@@ -207,7 +207,6 @@ struct SpanStamps {
 // Large-M kernel (sm24_prefill.hip): output columns per workgroup tile (N must be a
 // multiple) and its launcher.
 constexpr int kDecodeMaxM = 32;       // largest batch of one decode launch (two 16-row blocks)
-constexpr int kDecodeMidMaxM = 64;    // the mid-batch kernel reports the decode family up to here
 constexpr int kDecodeChunkMaxM = 96;  // largest batch run as several decode launches
 constexpr int kPreTileCols = 512;
 constexpr int kPreThreads = 512;  // one wave per 64-column chunk of the tile

@@ -888,6 +888,10 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
 // 2048x2048 3.6 against 4.5).  Where the 64-column tiles pass one round of the CUs, the
 // decode launches up to 32 rows keep their split tail, which callers that query the plan
 // expect (4096x22016 at M = 17 / 24 13.6 / 14.7 against 13.8 / 14.1).
+// 33-64 rows on narrow N once ran as a forced K split and a second launch that added the
+// partials; the plan is now free, and a split ends inside its launch (us per call, weights
+// cold, one box: 4096x4096 at M = 33 / 64 8.6 / 8.5 -> 6.8 / 6.6, 4096x6144 at 64 10.8 ->
+// 7.5, 8192x7936 17.7 -> 15.5, 11008x4096 14.2 -> 12.9, 28672x4096 25.3 -> 25.4).
 // MARLIN_HIP_MID=0 turns the kernel off (read once).
 constexpr int kMidMinM = 17, kMidMaxM = 192;
 // Narrow N (below 4096) leaves the large-M kernel a few workgroups that split K up to eight
@@ -910,22 +914,18 @@ MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
   MidShape best{0, 0, 0};
   if (!on || M < kMidMinM || M > mid_max_m(N, K) || K % 64 != 0 || (long long)M * K >= (1LL << 31)) return best;
   if ((M <= kDecodeMaxM && N / 64 > cus) || (K > 16384 && M > 64)) return best;
-  // Narrow N at 33-64 rows, K from 4096: the launches a query of the plan expects there are
-  // two, so K is split and a second launch adds the partials (4096x4096 at M = 64: one
-  // unsplit launch of 16-row tiles takes 6.9 us).
-  const bool two = !nosplit && M > kDecodeMaxM && M <= kDecodeMidMaxM && 2 * (N / 64) < cus && K >= 4096;
   double best_cost = 1e30;
   for (const Cand& c : cands) {
     if (N % (16 * c.ncb) != 0) continue;
     const long long tiles = (long long)(N / (16 * c.ncb)) * ((M + 16 * c.rb - 1) / (16 * c.rb));
-    for (int s = two ? 2 : 1; s <= (nosplit ? 1 : 8) && tiles * s <= cus; s++) {
+    for (int s = 1; s <= (nosplit ? 1 : 8) && tiles * s <= cus; s++) {
       if (s > 1 && K / 64 < 8 * s) break;
       const double x = (double)(tiles * s) / cus;
       double cost = 2.3 + (K / 64 / s + 7) / 8 * c.stage_us * (1 + 0.29 * (x - 0.75)) + 0.118 * c.ncb * c.rb;
       if (s > 1) cost += 1.13 + 8.0 * s * M * (double)N / 4.9e6;
       if (cost < best_cost) {
         best_cost = cost;
-        best = MidShape{c.ncb, c.rb, s, two};
+        best = MidShape{c.ncb, c.rb, s};
       }
     }
   }
@@ -992,7 +992,7 @@ void describe(int M, int N, int K, int sms, bool noalloc, int out[5]) {
     out[1] = N / (16 * d.ncb) * ((M + 16 * d.rb - 1) / (16 * d.rb)) * d.splits;
     out[2] = 512;
     out[3] = d.splits;
-    out[4] = d.two_launches ? 2 : 1;
+    out[4] = 1;
   } else if (kernel == KERNEL_DECODE) {
     const int mc = M < kDecodeMaxM ? M : kDecodeMaxM;
     DecodeShape d = decode_shape(mc, N, K, sms);
@@ -1073,7 +1073,6 @@ int run(int vf, int mf, const void* A, const void* B, const void* meta, void* C,
       err = get_scratch(dev, stream, tiles * d.splits * 256 * d.ncb * d.rb * sizeof(float), &p.counters, &p.partial);
       if (err != MARLIN_HIP_OK) return err;
       if (!p.counters) d = mid_plan(M, N, K, sms, true);  // capturing, and this stream has no scratch yet
-      else if (d.two_launches) p.counters = nullptr;
     }
     if (d.splits > 0) {
       p.splits = d.splits;

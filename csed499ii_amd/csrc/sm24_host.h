@@ -57,15 +57,12 @@ struct DecodeShape {
   int g = 1;          // tiles per workgroup (3: three 16-column tiles sharing resident rows)
 };
 
-// Tile of the mid-batch kernel (sm24_mid.h): 16 ncb columns x 16 rb rows, K splits, and
-// whether the splits' partials are added by a second launch (else by the last split).
+// Tile of the mid-batch kernel (sm24_mid.h): 16 ncb columns x 16 rb rows, and K splits.
 struct MidShape {
   int ncb, rb, splits;
-  bool two_launches = false;
 };
 struct GemmArgs;
-// Launch of the mid-batch kernel; a.splits > 1 without a.counters adds the partials in a
-// second launch.
+// Launch of the mid-batch kernel.
 hipError_t launch_mid(const GemmArgs& a, const MidShape& d, int vf, int mf, bool grouped, hipStream_t stream);
 
 // Padded batch of the decode kernel for M rows: 1, 4, 8, 16 or 32.

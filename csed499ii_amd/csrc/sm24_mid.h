@@ -22,8 +22,8 @@
 // than 8.
 //
 // us per call on one box, against the decode launches of up to 32 rows or the large-M
-// kernel: M = 64 7B qkv 18.9 -> 12.4, o 14.6 -> 8.4 (two launches), gate_up 21.3 -> 19.0,
-// down 20.2 -> 12.5, 70B o 24.3 -> 15.2, down 56.7 -> 33.7; M = 131 7B o 15.9 -> 8.6, 70B
+// kernel: M = 64 7B qkv 18.9 -> 12.4, o 14.6 -> 6.6, gate_up 21.3 -> 19.0,
+// down 20.2 -> 12.9, 70B o 24.3 -> 15.2, down 56.7 -> 33.7; M = 131 7B o 15.9 -> 8.6, 70B
 // qkv 35.9 -> 24.0; 2048x2048 at M = 96 17.4 -> 5.2.
 #pragma once
 #include "sm24_decode_dma.h"
@@ -350,10 +350,10 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
   }
   if (S == 1) return;
 
-  // ---- split-K: without counters a second launch (sm24_mid_reduce_kernel) adds the
-  // partials; else hand-off through the uncached scratch, as in the decode kernels: the
-  // last split to arrive adds all partials in split order and writes C ----
-  if (a.counters == nullptr) return;
+  // ---- split-K hand-off through the uncached scratch, as in the decode kernels: the last
+  // split to arrive adds all partials in split order and writes C.  It ends inside the
+  // launch: the calls of a stream share the scratch, and a launch of another host thread
+  // may lie between two of a call ----
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -378,27 +378,6 @@ __global__ __launch_bounds__(64 * kMidWaves) void sm24_mid_kernel(const void* B_
     }
     write_c(row, col, v);
   }
-}
-
-// Adds the S partials of every tile in split order and writes C: one thread per 4 columns
-// of a row.  TC and MB: columns and rows of the tiles.
-template <int TC, bool GROUPED>
-__global__ __launch_bounds__(256) void sm24_mid_reduce_kernel(GemmArgs a, int MB) {
-  const int N = a.N, M = a.M, S = a.splits, ntm = (M + MB - 1) / MB;
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  const int row = e / (N / 4), n = 4 * (e % (N / 4));
-  if (row >= M) return;
-  const int tile = n / TC * ntm + row / MB;
-  const float* p = a.partial + ((size_t)tile * S * MB + row % MB) * TC + n % TC;
-  float4_t v = *reinterpret_cast<const float4_t*>(p);
-  for (int z = 1; z < S; z++) v += *reinterpret_cast<const float4_t*>(p + (size_t)z * MB * TC);
-  half4_t o;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    o[i] = (_Float16)v[i];
-    if constexpr (!GROUPED) o[i] = o[i] * a.s[n + i];
-  }
-  *reinterpret_cast<half4_t*>(a.C + (size_t)row * N + n) = o;
 }
 
 // Launch of one operand format (sm24_mid.hip, sm24_mid_w3.hip, sm24_mid_m3.hip).

@@ -3,6 +3,8 @@ Llama-2-70B prefill sweep at full size, calls on two streams
 once, capture on a stream that has no split-K scratch yet, and the reference
 benchmark's own call sites (kernel_bench/bench.py).  Every check is against the CPU
 oracle, on column slices (every packed operand is self-contained per 64 columns)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -53,6 +55,44 @@ def test_prefill_llama70b_full_size(name, M):
     assert torch.equal(_mul(A, wt), C), "repeated prefill calls differ"
     chunks = N // 64
     check_slices(C, A.cpu().numpy(), t, (0, chunks // 2 - 1, chunks - 2), 2, f"prefill {name} M={M}")
+
+
+def _threads_on_one_stream(calls, rounds=40):
+    """Each of ``calls`` (a function that runs one call and returns its fresh output) in a
+    host thread of its own, all on the default stream at once: every output equals the
+    one of the same call run alone."""
+    refs = [c() for c in calls]
+    torch.cuda.synchronize()
+    outs = [[] for _ in calls]
+    start = threading.Barrier(len(calls))
+
+    def work(i):
+        for _ in range(rounds):
+            start.wait()
+            outs[i].append(calls[i]())
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(len(calls))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    torch.cuda.synchronize()
+    for ref, out in zip(refs, outs):
+        assert len(out) == rounds
+        for C in out:
+            assert torch.equal(C, ref)
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 4096, 4096), (64, 11008, 4096)])
+def test_threads_on_one_stream(M, K, N):
+    """Three host threads with their own weight and batch on one stream: calls share the
+    stream's split-K scratch, and none sees another's partials."""
+    calls = []
+    for i in range(3):
+        wt = synth.make_weight(K, N, 900 + i, 128, device=DEV)
+        A = synth.make_activation(M, K, 910 + i, device=DEV)
+        calls.append(lambda A=A, wt=wt: _mul(A, wt))
+    _threads_on_one_stream(calls)
 
 
 def test_two_streams_split_k_overlap():
