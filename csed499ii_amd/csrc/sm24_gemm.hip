@@ -415,6 +415,20 @@ int get_scratch(int dev, hipStream_t stream, size_t partial_bytes, uint32_t** co
 // grows, never freed.
 std::map<StreamKey, Scratch> g_stage;
 
+// Held from get_stage to the last launch of a call that uses the staging buffer: the
+// expansion and the kernel that reads it are launches of their own, and another host
+// thread's call on the same stream would otherwise fill the buffer between them.
+std::map<StreamKey, std::mutex> g_stage_order;
+
+std::unique_lock<std::mutex> stage_order(int dev, hipStream_t stream) {
+  std::mutex* order;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    order = &g_stage_order[StreamKey(dev, stream)];  // map nodes stay where they are
+  }
+  return std::unique_lock<std::mutex>(*order);
+}
+
 int get_stage(int dev, hipStream_t stream, size_t bytes, void** out) {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   Scratch& s = g_stage[StreamKey(dev, stream)];
@@ -1110,11 +1124,13 @@ int run(int vf, int mf, const void* A, const void* B, const void* meta, void* C,
     }
     return MARLIN_HIP_OK;
   }
+  std::unique_lock<std::mutex> staged;
   if (prefill_fits(M, N, K, VAL4, META4) && (vf != VAL4 || mf != META4)) {
     // 3-bit values or metadata at large M: expand them into the 4-bit layouts on this
     // stream, then the large-M kernel reads the expanded copy.
     const size_t vbytes = vf == VAL3 ? (size_t)K * N / 4 : 0, mbytes = mf == META3 ? (size_t)K * N / 8 : 0;
     void* stage = nullptr;
+    staged = stage_order(dev, stream);
     err = get_stage(dev, stream, vbytes + mbytes, &stage);
     if (err != MARLIN_HIP_OK) return err;
     if (vf == VAL3) {
@@ -1312,6 +1328,7 @@ int run_native(const void* A, const void* W, const void* X, void* C, const void*
     // stream) and run the reference-layout kernels on it.
     const size_t vb = (size_t)K * N / 4, mb = (size_t)K * N / 8, sb = (size_t)(grouped ? K / 128 : 1) * N * 2;
     void* stage = nullptr;
+    const std::unique_lock<std::mutex> staged = stage_order(dev, stream);
     err = get_stage(dev, stream, vb + mb + sb, &stage);
     if (err != MARLIN_HIP_OK) return err;
     char* b = static_cast<char*>(stage);

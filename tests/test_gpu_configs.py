@@ -95,6 +95,32 @@ def test_threads_on_one_stream(M, K, N):
     _threads_on_one_stream(calls)
 
 
+@pytest.mark.parametrize("op,M,K,N", [("w3", 300, 2048, 8192), ("meta3", 131, 4096, 22016),
+                                      ("native", 24, 4096, 4096), ("native", 300, 2048, 8192)])
+def test_threads_on_one_stream_staged(op, M, K, N):
+    """Three host threads on one stream, each expanding or unpacking its own weight into
+    the stream's staging buffer before the GEMM reads it there."""
+    calls = []
+    for i in range(3):
+        wt = synth.make_weight(K, N, 920 + i, 128, bits=3 if op == "w3" else 4, device=DEV)
+        A = synth.make_activation(M, K, 930 + i, device=DEV)
+        meta3 = marlin.pack_meta3(wt["meta"].reshape(-1)) if op == "meta3" else None
+        native = marlin.pack_native(wt["B"], wt["meta"], wt["s"]) if op == "native" else None
+
+        def call(A=A, wt=wt, meta3=meta3, native=native):
+            C = torch.empty((M, N), dtype=torch.half, device=DEV)
+            if op == "w3":
+                marlin.mul_2_4_w3(A, wt["B"], wt["meta"], C, wt["s"], _ws(N))
+            elif op == "meta3":
+                marlin.mul_2_4_meta3(A, wt["B"], meta3, C, wt["s"], _ws(N))
+            else:
+                marlin.mul_2_4_native(A, native[0], native[1], C, native[2])
+            return C
+
+        calls.append(call)
+    _threads_on_one_stream(calls)
+
+
 def test_two_streams_split_k_overlap():
     """Two layers on two same-priority streams, both planned with split-K (gate_up
     4096x22016 at M = 24 splits in two, Llama-2-70B qkv 8192x10240 at M = 4 in four),

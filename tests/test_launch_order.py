@@ -28,3 +28,17 @@ def test_split_k_hand_off_in_one_launch(fake, op, M, K, N):
     call = [op, M, K, N, 128, 256]
     assert [x["kernel"] for x in launches(fake, [[call]])] == ["sm24_mid_kernel"]
     assert_calls_whole(fake, call, 1)
+
+
+@pytest.mark.parametrize("op,M,K,N,kernels", [
+    ("w3", 512, 4096, 4096, ["w3_to_w4_kernel", "sm24_prefill_kernel"]),
+    ("meta3", 131, 4096, 22016, ["meta3_unpack_kernel", "sm24_prefill_kernel"]),
+    ("native", 24, 4096, 4096, ["native_unpack_values_kernel", "native_unpack_meta_kernel", "sm24_mid_kernel"]),
+    ("native", 600, 4096, 4096, ["native_unpack_values_kernel", "native_unpack_meta_kernel", "sm24_prefill_kernel"]),
+])
+def test_staged_operands(fake, op, M, K, N, kernels):
+    """Operands expanded into the stream's staging buffer: the expansion and the kernel that
+    reads it follow each other."""
+    call = [op, M, K, N, 128, 256]
+    assert [x["kernel"] for x in launches(fake, [[call]])] == kernels
+    assert_calls_whole(fake, call, len(kernels))
