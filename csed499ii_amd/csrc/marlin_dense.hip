@@ -325,7 +325,7 @@ DenseMidShape dense_mid_plan(int M, int N, int K, int cus, bool nosplit, double*
     if (N % (64 * c.nch) != 0) continue;
     const long long tiles = (long long)(N / (64 * c.nch)) * ((M + 16 * c.rb - 1) / (16 * c.rb));
     for (int s = 1; s <= (nosplit ? 1 : 8); s++) {
-      if (s > 1 && (tiles * s > cus || K / 64 < 8 * s)) break;
+      if (s > 1 && (tiles * s > cus || K / 64 < 8 * s || (size_t)tiles * sizeof(uint32_t) > kCounterBytes)) break;
       const double x = (double)(tiles * s) / cus;
       const double rounds = x <= 1 ? 1 : (double)((tiles * s + cus - 1) / cus);
       const double share = x > 1 && c.nch * c.rb <= 2 ? 0.89 : 1.0;

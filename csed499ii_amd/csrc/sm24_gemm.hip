@@ -548,9 +548,11 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
     if (forced_chunks && c.chunks != forced_chunks) continue;
     const int tiles = ((N + 64 * c.chunks - 1) / (64 * c.chunks)) * ((M + c.rows - 1) / c.rows);
     const int cmax_s = max_s / c.groups > 0 ? max_s / c.groups : 1;
-    if (forced && !nosplit) return PrefillPlan{c.rows, forced < cmax_s ? forced : cmax_s, tiles, c.chunks};
+    const bool counted = (size_t)tiles * sizeof(uint32_t) <= kCounterBytes;  // one arrival counter per tile
+    if (forced && !nosplit)
+      return PrefillPlan{c.rows, !counted ? 1 : forced < cmax_s ? forced : cmax_s, tiles, c.chunks};
     for (int s = 1; s <= 8 && s <= cmax_s; s++) {
-      if (s > 1 && (size_t)tiles * sizeof(uint32_t) > kCounterBytes) break;  // one arrival counter per tile
+      if (s > 1 && !counted) break;
       const long long wgs = (long long)tiles * s, full = wgs / cus, tail = wgs - full * cus;
       double cost = ((double)full * prefill_step_us(1.0) + (tail ? prefill_step_us((double)tail / cus) : 0.0)) *
                     c.hscale * nks / (s * c.groups);
@@ -933,7 +935,7 @@ MidShape mid_plan(int M, int N, int K, int cus, bool nosplit) {
     if (N % (16 * c.ncb) != 0) continue;
     const long long tiles = (long long)(N / (16 * c.ncb)) * ((M + 16 * c.rb - 1) / (16 * c.rb));
     for (int s = 1; s <= (nosplit ? 1 : 8) && tiles * s <= cus; s++) {
-      if (s > 1 && K / 64 < 8 * s) break;
+      if (s > 1 && (K / 64 < 8 * s || (size_t)tiles * sizeof(uint32_t) > kCounterBytes)) break;
       const double x = (double)(tiles * s) / cus;
       double cost = 2.3 + (K / 64 / s + 7) / 8 * c.stage_us * (1 + 0.29 * (x - 0.75)) + 0.118 * c.ncb * c.rb;
       if (s > 1) cost += 1.13 + 8.0 * s * M * (double)N / 4.9e6;

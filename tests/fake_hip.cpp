@@ -1,5 +1,5 @@
 // A HIP runtime that launches nothing: each kernel launch is only written down (kernel,
-// grid, K splits of the mid-batch kernels, host thread, stream).  Loaded into a process
+// grid, K splits of the mid-batch and large-M kernels, host thread).  Loaded into a process
 // of its own ahead of libmarlin_hip.so, it shows on the CPU which kernels a call runs and
 // in which order the launches of several host threads reach a stream.  Every launch
 // takes a millisecond, so that threads that may interleave do.
@@ -22,7 +22,7 @@ namespace {
 struct Launch {
   std::string kernel;
   unsigned grid, block;
-  int splits;  // of the mid-batch kernels (else 0)
+  int splits;  // of the mid-batch and large-M kernels (else 0)
   int caller;  // set by fake_hip_caller on the calling thread
 };
 std::mutex mu;
@@ -88,6 +88,9 @@ int hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, size_t, 
     // their arguments: A, B, s, M, N, K, splits and B, meta, s, A, zeros, M, N, K, splits
     if (l.kernel.find("marlin_dense_mid_kernel") != std::string::npos) l.splits = *static_cast<int*>(args[6]);
     if (l.kernel.find("sm24_mid_kernel") != std::string::npos) l.splits = *static_cast<int*>(args[8]);
+    // its GemmArgs: six pointers, M, N, K, splits
+    if (l.kernel.find("sm24_prefill_kernel") != std::string::npos)
+      l.splits = *reinterpret_cast<int*>(static_cast<char*>(args[0]) + 6 * sizeof(void*) + 3 * sizeof(int));
     launches.push_back(l);
   }
   const timespec ms{0, 1000000};

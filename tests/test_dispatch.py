@@ -1,0 +1,31 @@
+"""Which kernels the calls run and with which K splits, on the CPU (tests/launches.py)."""
+import pytest
+
+from csed499ii_amd import _lib
+from tests.launches import build_fake, launches
+
+COUNTERS = 64 * 1024 // 4  # arrival counters of a stream's split-K scratch
+
+
+@pytest.fixture(scope="module")
+def fake(built_lib, tmp_path_factory):
+    return build_fake(tmp_path_factory.mktemp("fake_hip"))
+
+
+@pytest.mark.parametrize("op,M,K,N", [("2_4", 192, 1024, 524288), ("w3", 17, 1 << 17, 576 << 10), ("2_4", 33, 16384, 4096),
+                                      ("dense", 2048, 1024, 16384), ("dense", 1, 16384, 1040 << 10)])
+@pytest.mark.parametrize("sms", [256, 1 << 15, 1 << 20, (1 << 31) - 1])
+def test_splits_within_counters(fake, op, M, K, N, sms):
+    """Any number of compute units a caller names: a call whose K is split has an arrival
+    counter for every tile."""
+    for x in launches(fake, [[[op, M, K, N, 128, sms]]]):
+        assert x["splits"] <= 1 or x["grid"] // x["splits"] <= COUNTERS, x
+
+
+@pytest.mark.parametrize("rows", ["64", "96", "128"])
+def test_forced_splits_within_counters(fake, rows):
+    """Forced K splits of the large-M kernel, on every tile height."""
+    env = {"MARLIN_HIP_PREFILL_SPLITS": "2", "MARLIN_HIP_PREFILL_ROWS": rows}
+    (x,) = launches(fake, [[["2_4", 4096, 2048, 131072, 128, 256]]], env)
+    assert x["kernel"] == "sm24_prefill_kernel"
+    assert x["splits"] <= 1 or x["grid"] // x["splits"] <= COUNTERS, x
