@@ -242,15 +242,19 @@ hipError_t launch_dense_t(const DenseArgs& a, dim3 grid, hipStream_t stream) {
 
 // Large-M path (marlin_dense_prefill_kernel): K a multiple of 128 (whole scale groups, an
 // even number of 64-deep k-steps), N of its 512-column tile or of half of it (the last tile
-// is then half empty).  32-bit operand offsets; from MARLIN_HIP_DENSE_PREFILL_MIN_M rows
-// (default 65).
-bool dense_prefill_fits(int M, int N, int K) {
-  static const int forced_min_m = [] {
+// is then half empty).  32-bit operand offsets; from 65 rows.
+// MARLIN_HIP_DENSE_PREFILL_MIN_M (>= 1) replaces the threshold, and then every call from it
+// on runs this kernel, whatever dense_mid_fits estimates.
+int dense_prefill_forced_min_m() {
+  static const int v = [] {
     const char* e = getenv("MARLIN_HIP_DENSE_PREFILL_MIN_M");
     const int x = e ? atoi(e) : 0;
     return x >= 1 ? x : 0;
   }();
-  const int min_m = forced_min_m ? forced_min_m : 65;
+  return v;
+}
+bool dense_prefill_fits(int M, int N, int K) {
+  const int min_m = dense_prefill_forced_min_m() ? dense_prefill_forced_min_m() : 65;
   return M >= min_m && N % (kDpTileCols / 2) == 0 && K % 128 == 0 && (long long)M * K < (1LL << 31) - 2048 &&
          (long long)K * N < (1LL << 33);
 }
@@ -353,6 +357,7 @@ constexpr int kDenseMidMaxM = 2048;
 bool dense_mid_fits(int M, int N, int K, int cus) {
   if (M > kDenseMidMaxM || (long long)M * K >= (1LL << 31)) return false;
   if (!dense_prefill_fits(M, N, K)) return true;
+  if (dense_prefill_forced_min_m()) return false;
   const int tiles = ((N + kDpTileCols - 1) / kDpTileCols) * ((M + kDpRows - 1) / kDpRows);
   double mid = 0.0, pre = 0.0;
   dense_mid_plan(M, N, K, cus, false, &mid);

@@ -865,8 +865,8 @@ hipError_t launch_decode(const GemmArgs& a, DecodeShape d, int vf, int mf, bool 
 // 64 the decode launches win for 7B o, down and qkv: 7B o 13.6 / 15.0 against 19.6 /
 // 20.0 us); above the decode launches' 96 rows for narrower N (against the multi-block
 // kernel: 4096x768 at M = 160 43.3 -> 20.6 us, 4096x2816 31.0 -> 20.9, 8192x768 47.1 ->
-// 24.4).  MARLIN_HIP_PREFILL_MIN_M (>= 1) replaces the
-// threshold.
+// 24.4).  MARLIN_HIP_PREFILL_MIN_M (>= 1) replaces the threshold, ahead of the mid-batch
+// kernel's rule.
 int prefill_min_m(int N, int K) {
   // the widest N at long K already from 17 rows (70B gate_up 8192x57344 at M = 24 /
   // 32: 49.5 / 50.3 against 58.8 / 67.3 us; at M = 16 49.5 against 49.0)
@@ -875,13 +875,16 @@ int prefill_min_m(int N, int K) {
   return N >= 4096 ? 65 : kDecodeChunkMaxM + 1;
 }
 bool prefill_n(int N) { return N % kPreTileCols == 0 || (N % (kPreTileCols / 2) == 0 && N >= 2 * kPreTileCols); }
-bool prefill_fits(int M, int N, int K, int vf, int mf) {
-  static const int forced_min_m = [] {
+int prefill_forced_min_m() {
+  static const int v = [] {
     const char* e = getenv("MARLIN_HIP_PREFILL_MIN_M");
     const int x = e ? atoi(e) : 0;
     return x >= 1 ? x : 0;
   }();
-  const int min_m = forced_min_m ? forced_min_m : prefill_min_m(N, K);
+  return v;
+}
+bool prefill_fits(int M, int N, int K, int vf, int mf) {
+  const int min_m = prefill_forced_min_m() ? prefill_forced_min_m() : prefill_min_m(N, K);
   return vf == VAL4 && mf == META4 && M >= min_m && prefill_n(N) && K % 128 == 0 &&
          (long long)M * K < (1LL << 31) - 2048 && (long long)K * N < (1LL << 34);
 }
@@ -986,8 +989,9 @@ enum : int { KERNEL_DECODE = 0, KERNEL_PREFILL = 1, KERNEL_GENERAL = 2, KERNEL_D
 // against 49.7 us for the general kernel); the large-M kernel where it fits; the
 // general kernel otherwise.
 int kernel_for(int M, int N, int K, int cus, bool nosplit) {
-  if (mid_fits(M, N, K, cus, nosplit)) return KERNEL_MID;
-  if (prefill_fits(M, N, K, VAL4, META4)) return KERNEL_PREFILL;
+  const bool prefill = prefill_fits(M, N, K, VAL4, META4);
+  if (!(prefill && prefill_forced_min_m()) && mid_fits(M, N, K, cus, nosplit)) return KERNEL_MID;
+  if (prefill) return KERNEL_PREFILL;
   return M <= kDecodeChunkMaxM ? KERNEL_DECODE : KERNEL_GENERAL;
 }
 

@@ -29,3 +29,16 @@ def test_forced_splits_within_counters(fake, rows):
     (x,) = launches(fake, [[["2_4", 4096, 2048, 131072, 128, 256]]], env)
     assert x["kernel"] == "sm24_prefill_kernel"
     assert x["splits"] <= 1 or x["grid"] // x["splits"] <= COUNTERS, x
+
+
+@pytest.mark.parametrize("op,env,kernel", [
+    ("2_4", {"MARLIN_HIP_PREFILL_MIN_M": "48"}, "sm24_prefill_kernel"),
+    ("w3", {"MARLIN_HIP_PREFILL_MIN_M": "48"}, "sm24_prefill_kernel"),
+    ("dense", {"MARLIN_HIP_DENSE_PREFILL_MIN_M": "48"}, "marlin_dense_prefill_kernel"),
+])
+def test_prefill_min_m_switch(fake, op, env, kernel):
+    """The smallest batch of the large-M kernels, where it is set: every call they can take
+    from it on, none below it."""
+    for M, K, N in ((48, 4096, 4096), (64, 2048, 1024), (160, 4096, 12288), (1000, 1024, 2048)):
+        assert launches(fake, [[[op, M, K, N, 128, 256]]], env)[-1]["kernel"] == kernel, (M, K, N)
+        assert launches(fake, [[[op, 47, K, N, 128, 256]]], env)[-1]["kernel"] != kernel, (47, K, N)
