@@ -538,8 +538,9 @@ PrefillPlan prefill_plan(int M, int N, int K, int cus, bool nosplit) {
                         {128, kPreNarrowChunks, 1, kPreNarrowStep},
                         {64, kPreNarrowChunks, 2, 0.69},
                         {96, kPreNarrowChunks, 2, 1.15}};
-  // Up to kPreGroupMaxM rows the two-group tiles replace the 64-row 512-column ones.
-  const bool groups = (M <= kPreGroupMaxM || forced_rows) && nks >= 16 && forced_chunks != kPreChunks;
+  // Up to kPreGroupMaxM rows the two-group tiles replace the 64-row 512-column ones, unless
+  // a forced width asks for the other tiles.
+  const bool groups = (M <= kPreGroupMaxM || forced_rows) && nks >= 16 && !forced_chunks;
   for (const Cand& c : cands) {
     if (c.groups == 1 && (c.chunks == kPreNarrowChunks) != (forced_chunks == kPreNarrowChunks)) continue;
     if (c.groups > 1 && !groups) continue;

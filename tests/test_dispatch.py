@@ -42,3 +42,13 @@ def test_prefill_min_m_switch(fake, op, env, kernel):
     for M, K, N in ((48, 4096, 4096), (64, 2048, 1024), (160, 4096, 12288), (1000, 1024, 2048)):
         assert launches(fake, [[[op, M, K, N, 128, 256]]], env)[-1]["kernel"] == kernel, (M, K, N)
         assert launches(fake, [[[op, 47, K, N, 128, 256]]], env)[-1]["kernel"] != kernel, (47, K, N)
+
+
+@pytest.mark.parametrize("chunks,block", [("4", 256), ("8", 512)])
+def test_prefill_chunks_switch(fake, chunks, block):
+    """4: every large-M call on the narrow tile of four waves; 8: on 512-column tiles of
+    eight, also at the batches of the two-group tiles."""
+    for M, K, N in ((80, 4096, 22016), (131, 4096, 22016), (192, 8192, 16384), (1000, 4096, 8192)):
+        (x,) = launches(fake, [[["2_4", M, K, N, 128, 256]]], {"MARLIN_HIP_PREFILL_CHUNKS": chunks})
+        assert x["kernel"] == "sm24_prefill_kernel" and x["block"] == block, (M, K, N, x)
+        assert f"ELi{chunks}ELi1EE" in x["symbol"], x  # chunks, one k-group
