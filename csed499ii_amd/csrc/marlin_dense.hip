@@ -270,8 +270,8 @@ int dense_prefill_splits(int tiles, int nks, int cus, double* estimate = nullptr
     const int x = e ? atoi(e) : 0;
     return x >= 1 && x <= 16 ? x : 0;
   }();
-  const int max_s = nks / 8;  // at least eight k-steps per split
-  if (forced) return forced < max_s ? forced : (max_s > 0 ? max_s : 1);
+  const int max_s = nks / 8 > 0 ? nks / 8 : 1;  // at least eight k-steps per split
+  if (forced) return forced < max_s ? forced : max_s;
   const double step_us = 1.3, exchange_bytes_per_us = 2.5e6;
   int best_s = 1;
   double best = 1e30;
@@ -284,8 +284,8 @@ int dense_prefill_splits(int tiles, int nks, int cus, double* estimate = nullptr
       best_s = s;
     }
   }
-  if ((size_t)tiles * sizeof(uint32_t) > kCounterBytes) best_s = 1;
   if (estimate) *estimate = best;
+  if ((size_t)tiles * sizeof(uint32_t) > kCounterBytes) best_s = 1;
   return best_s;
 }
 
@@ -351,8 +351,12 @@ DenseMidShape dense_mid_plan(int M, int N, int K, int cus, bool nosplit, double*
 // clearly lower.  Over the sweep above and 90 random shapes at 400-4096 rows this keeps
 // the faster of the two or one within a few per cent of it up to 2048 rows (large-M ->
 // this kernel, us: 943x1792x3584 43.7 -> 28.0, 768x11008x1536 68.1 -> 36.9, 1168x1280x1280
-// 34.3 -> 12.2); beyond, two calls lost (3257x10752x2560 201.9 -> 224.3).  32-bit
-// activation offsets.
+// 34.3 -> 12.2); beyond, two calls lost (3257x10752x2560 201.9 -> 224.3).  Below K = 512 the
+// large-M kernel's fixed cost is most of its time, and the estimate has none of it: both
+// kernels on 90 calls of K 128-384, N 1024-57344 and 65-2048 rows, one box (us, mid /
+// large-M: 128x4096 at 512 rows 6.7 / 12.3, at 2048 22.2 / 14.4; 384x22016 at 131 15.4 /
+// 19.1, at 512 42.1 / 21.6; 256x57344 at 2048 302 / 144); the rule takes the slower of the
+// pair once (384x57344 at 65 rows, 20.8 / 16.4).  32-bit activation offsets.
 constexpr int kDenseMidMaxM = 2048;
 bool dense_mid_fits(int M, int N, int K, int cus) {
   if (M > kDenseMidMaxM || (long long)M * K >= (1LL << 31)) return false;
@@ -362,7 +366,7 @@ bool dense_mid_fits(int M, int N, int K, int cus) {
   double mid = 0.0, pre = 0.0;
   dense_mid_plan(M, N, K, cus, false, &mid);
   dense_prefill_splits(tiles, K / 64, cus, &pre);
-  return mid < 0.82 * (pre + 6.0);
+  return mid < 0.82 * (pre + (K < 512 ? 15.5 : 6.0));
 }
 
 int run_dense_mid(const void* A, const void* B, void* C, const void* s, int M, int N, int K, bool grouped, int dev,

@@ -52,3 +52,14 @@ def test_prefill_chunks_switch(fake, chunks, block):
         (x,) = launches(fake, [[["2_4", M, K, N, 128, 256]]], {"MARLIN_HIP_PREFILL_CHUNKS": chunks})
         assert x["kernel"] == "sm24_prefill_kernel" and x["block"] == block, (M, K, N, x)
         assert f"ELi{chunks}ELi1EE" in x["symbol"], x  # chunks, one k-group
+
+
+@pytest.mark.parametrize("K", [128, 256, 384])
+def test_dense_short_k(fake, K):
+    """Dense calls of fewer than eight k-steps run the faster of the two kernels, as longer
+    K do: the large-M kernel on much work, the mid-batch one on little."""
+    for M, N, kernel in ((2048, 57344, "marlin_dense_prefill_kernel"), (512, 22016, "marlin_dense_prefill_kernel"),
+                         (131, 57344, "marlin_dense_prefill_kernel"), (2048, 4096, "marlin_dense_prefill_kernel"),
+                         (512, 4096, "marlin_dense_mid_kernel"), (131, 11008, "marlin_dense_mid_kernel"),
+                         (2048, 1024, "marlin_dense_mid_kernel"), (64, 57344, "marlin_dense_mid_kernel")):
+        assert [x["kernel"] for x in launches(fake, [[["dense", M, K, N, 128, 256]]])] == [kernel], (M, K, N)
