@@ -263,7 +263,7 @@ bool dense_prefill_fits(int M, int N, int K) {
 // one workgroup per CU times the k-steps per split, plus the partial exchange (each
 // split stores a 256 KiB fp32 tile), at ~1.3 us per 64-deep k-step of a tile (32
 // MFMAs per wave) and ~2.5 TB/s for the exchange.  MARLIN_HIP_DENSE_PREFILL_SPLITS
-// forces a count.  *estimate: the model's time, us.
+// forces a count.  *estimate: the model's time of its own choice, us, forced or not.
 int dense_prefill_splits(int tiles, int nks, int cus, double* estimate = nullptr) {
   static const int forced = [] {
     const char* e = getenv("MARLIN_HIP_DENSE_PREFILL_SPLITS");
@@ -271,7 +271,6 @@ int dense_prefill_splits(int tiles, int nks, int cus, double* estimate = nullptr
     return x >= 1 && x <= 16 ? x : 0;
   }();
   const int max_s = nks / 8 > 0 ? nks / 8 : 1;  // at least eight k-steps per split
-  if (forced) return forced < max_s ? forced : max_s;
   const double step_us = 1.3, exchange_bytes_per_us = 2.5e6;
   int best_s = 1;
   double best = 1e30;
@@ -285,6 +284,7 @@ int dense_prefill_splits(int tiles, int nks, int cus, double* estimate = nullptr
     }
   }
   if (estimate) *estimate = best;
+  if (forced) best_s = forced < max_s ? forced : max_s;
   if ((size_t)tiles * sizeof(uint32_t) > kCounterBytes) best_s = 1;
   return best_s;
 }

@@ -63,3 +63,18 @@ def test_dense_short_k(fake, K):
                          (512, 4096, "marlin_dense_mid_kernel"), (131, 11008, "marlin_dense_mid_kernel"),
                          (2048, 1024, "marlin_dense_mid_kernel"), (64, 57344, "marlin_dense_mid_kernel")):
         assert [x["kernel"] for x in launches(fake, [[["dense", M, K, N, 128, 256]]])] == [kernel], (M, K, N)
+
+
+def test_dense_prefill_splits_switch(fake):
+    """The switch forces the large-M kernel's K splits (at most one per eight k-steps, one
+    arrival counter per tile) and leaves the choice of kernel alone."""
+    calls = [["dense", M, K, N, 128, 256] for M in (65, 131, 512, 2048, 4096)
+             for K, N in ((4096, 4096), (11008, 4096), (4096, 22016), (256, 11008), (1024, 1 << 20))]
+    free = launches(fake, [calls])
+    forced = launches(fake, [calls], {"MARLIN_HIP_DENSE_PREFILL_SPLITS": "3"})
+    assert [x["kernel"] for x in free] == [x["kernel"] for x in forced]
+    for (_, M, K, N, *_), x in zip(calls, forced):
+        if x["kernel"] == "marlin_dense_prefill_kernel":
+            tiles = -(-N // 512) * -(-M // 128)
+            s = min(3, max(1, K // 512)) if tiles <= COUNTERS else 1
+            assert x["grid"] == tiles * s, (M, K, N, x)
