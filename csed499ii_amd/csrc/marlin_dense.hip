@@ -315,35 +315,55 @@ int run_dense_prefill(const void* A, const void* B, void* C, const void* s, int 
 // best of each call): a fixed cost, the stages of a wave at the tile's measured stage time
 // per round of workgroups over the CUs (less for the small tiles, two of which share a CU),
 // the reduction in LDS, the codes' bytes, and for a split the exchange of the fp32 partials
-// (only up to one workgroup per CU).  *cost in us.
+// (only up to one workgroup per CU).  *cost: the model's time of its own choice, us.
+// MARLIN_HIP_DENSE_SPLITS (1-16, at most K / 256) forces the K splits, on the tile that the
+// model then has the fastest.
 DenseMidShape dense_mid_plan(int M, int N, int K, int cus, bool nosplit, double* cost) {
+  static const int forced = [] {
+    const char* e = getenv("MARLIN_HIP_DENSE_SPLITS");
+    const int x = e ? atoi(e) : 0;
+    return x >= 1 && x <= 16 ? x : 0;
+  }();
   struct Cand {
     int nch, rb;
     double stage_us;
   };
   static const Cand cands[] = {{1, 1, 0.60}, {1, 2, 0.72}, {1, 3, 0.92}, {1, 4, 1.06}, {1, 5, 1.26},
                                {2, 1, 1.07}, {2, 2, 1.27}, {2, 3, 1.51}, {2, 4, 1.73}};
-  DenseMidShape best{1, 1, 1};
-  double best_cost = 1e30;
+  DenseMidShape best{1, 1, 1}, fbest{0, 0, 0};
+  double best_cost = 1e30, fbest_cost = 1e30;
   for (const Cand& c : cands) {
     if (N % (64 * c.nch) != 0) continue;
     const long long tiles = (long long)(N / (64 * c.nch)) * ((M + 16 * c.rb - 1) / (16 * c.rb));
-    for (int s = 1; s <= (nosplit ? 1 : 8); s++) {
-      if (s > 1 && (tiles * s > cus || K / 64 < 8 * s || (size_t)tiles * sizeof(uint32_t) > kCounterBytes)) break;
+    const bool counted = (size_t)tiles * sizeof(uint32_t) <= kCounterBytes;  // one arrival counter per tile
+    auto us = [&](int s) {
       const double x = (double)(tiles * s) / cus;
       const double rounds = x <= 1 ? 1 : (double)((tiles * s + cus - 1) / cus);
       const double share = x > 1 && c.nch * c.rb <= 2 ? 0.89 : 1.0;
       const double f = share * rounds * (1 + 0.295 * (x / rounds - 0.75));
       double t = 2.7 + (K / 64 / s + 7) / 8 * c.stage_us * f + 0.50 * c.nch * c.rb * rounds + 2.8e-8 * K * (double)N;
       if (s > 1) t += 1.44 + 8.0 * s * M * (double)N / 7.5e6;
+      return t;
+    };
+    for (int s = 1; s <= (nosplit ? 1 : 8); s++) {
+      if (s > 1 && (tiles * s > cus || K / 64 < 8 * s || !counted)) break;
+      const double t = us(s);
       if (t < best_cost) {
         best_cost = t;
         best = DenseMidShape{c.nch, c.rb, s};
       }
     }
+    if (forced && !nosplit) {
+      const int smax = K / 256 > 0 && counted ? K / 256 : 1, s = forced < smax ? forced : smax;
+      const double t = us(s);
+      if (t < fbest_cost) {
+        fbest_cost = t;
+        fbest = DenseMidShape{c.nch, c.rb, s};
+      }
+    }
   }
   if (cost) *cost = best_cost;
-  return best;
+  return fbest.splits > 0 ? fbest : best;
 }
 
 // Whether a call runs the decode- and mid-batch kernel: up to 64 rows always, up to 2048

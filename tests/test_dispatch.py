@@ -78,3 +78,19 @@ def test_dense_prefill_splits_switch(fake):
             tiles = -(-N // 512) * -(-M // 128)
             s = min(3, max(1, K // 512)) if tiles <= COUNTERS else 1
             assert x["grid"] == tiles * s, (M, K, N, x)
+
+
+@pytest.mark.parametrize("splits", [1, 3, 16])
+def test_dense_splits_switch(fake, splits):
+    """The switch forces the K splits of the dense decode- and mid-batch kernel (at most
+    one per 256 of K, one arrival counter per tile) and leaves the choice of kernel alone."""
+    calls = [["dense", M, K, N, 128, 256] for M in (1, 16, 64, 131, 2048)
+             for K, N in ((4096, 4096), (11008, 4096), (1152, 22016), (256, 11008), (8192, 1 << 21))]
+    free = launches(fake, [calls])
+    forced = launches(fake, [calls], {"MARLIN_HIP_DENSE_SPLITS": str(splits)})
+    assert [x["kernel"] for x in free] == [x["kernel"] for x in forced]
+    for (_, M, K, N, *_), x in zip(calls, forced):
+        if x["kernel"] == "marlin_dense_mid_kernel":
+            assert x["splits"] in (min(splits, K // 256), 1)
+            assert x["splits"] == 1 or x["grid"] // x["splits"] <= COUNTERS, (M, K, N, x)
+            assert x["splits"] > 1 or splits == 1 or K == 256 or N > 1 << 20, (M, K, N, x)
