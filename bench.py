@@ -130,23 +130,18 @@ def kernel_of(c) -> str:
     """The kernel the library dispatches a call to: the lane-native kernel for the
     lane-native layout, the dense kernels for the dense op, else the first launch's
     kernel of the library's own plan (``marlin.plan_2_4``: the register-ring decode
-    kernel at 1-8 padded rows, the LDS-DMA decode kernel up to 32, the large-M
-    kernel, or the general one).  From 17 to 192 rows the plan names the family of the
-    batch, and the mid-batch kernel runs where one round of its workgroups covers the
-    call; so do the dense kernels above 64 rows: both names are given there."""
+    kernel at 1-8 padded rows, the LDS-DMA decode kernel up to 32, the mid-batch kernel,
+    the large-M kernel, or the general one).  The dense op has no plan query: above 64
+    rows both kernels that its planner chooses from are named."""
     if getattr(c, "native", False):
         return "sm24::sm24_native_decode_kernel"
     if getattr(c, "bits", None) == "dense":
         if c.M > 64:
             return "sm24::marlin_dense_prefill_kernel or sm24::marlin_dense_mid_kernel"
         return "sm24::marlin_dense_mid_kernel"
-    plan = marlin.plan_2_4(c.M, c.K, c.N, 128)
-    kind = plan["kernel"]
-    if 17 <= c.M <= 192 and plan["threads"] == 512:
-        return {"decode_dma": "sm24::sm24_decode_dma_kernel", "large_m": "sm24::sm24_prefill_kernel"}[kind] + \
-            " or sm24::sm24_mid_kernel"
+    kind = marlin.plan_2_4(c.M, c.K, c.N, 128)["kernel"]
     return {"decode": "sm24::sm24_decode_kernel", "decode_dma": "sm24::sm24_decode_dma_kernel",
-            "large_m": "sm24::sm24_prefill_kernel", "general": "sm24::sm24_gemm_kernel"}[kind]
+            "mid": "sm24::sm24_mid_kernel", "large_m": "sm24::sm24_prefill_kernel", "general": "sm24::sm24_gemm_kernel"}[kind]
 
 
 def dense_fn(A, B, meta, C, s, ws):

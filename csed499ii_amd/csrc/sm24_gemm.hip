@@ -855,8 +855,8 @@ hipError_t launch_decode(const GemmArgs& a, DecodeShape d, int vf, int mf, bool 
 // its 64-deep k-steps, N of its 512-column tile or, from 1024 columns, of half of it (the
 // last tile is then half empty; against the multi-block kernel, us per call, one box:
 // 4096x11008 at M = 100 / 777 / 2000 65.6 / 300 / 709 -> 23.6 / 54 / 119, 4096x1280 at
-// M = 160 / 777 32.3 / 51.7 -> 21.3 / 24.3; 768 columns keep the multi-block kernel, as
-// callers that query the plan expect), from a batch threshold measured on
+// M = 160 / 777 32.3 / 51.7 -> 21.3 / 24.3; 768 columns run the mid-batch kernel up to
+// 1024 rows and have not been measured here above that), from a batch threshold measured on
 // MI355X against decode launches of <= 32 rows (Llama-2-7B and -70B shapes, M in
 // 48..192, the planner's 64- or 128-row tiles): from M = 33 for the widest N (7B
 // gate_up 4096x22016 at M = 48 / 64: 23.5 / 23.3 against 28.1 / 34.0 us) and for long
@@ -906,8 +906,8 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
 // 13.6 -> 11.8 / 12.0 / 12.4, down 28.6 / 31.7 / 34.1 -> 24.7 / 25.0 / 25.7, 2048x2048 5.8 /
 // 5.9 / 6.0 -> 4.5), but not at 12 rows, where those stage 16 (7B qkv 8.1 against 9.1,
 // 2048x2048 3.6 against 4.5).  Where the 64-column tiles pass one round of the CUs, the
-// decode launches up to 32 rows keep their split tail, which callers that query the plan
-// expect (4096x22016 at M = 17 / 24 13.6 / 14.7 against 13.8 / 14.1).
+// decode launches up to 32 rows keep their split tail: no clear gain (4096x22016 at M = 17 /
+// 24 13.6 / 14.7 against 13.8 / 14.1).
 // 33-64 rows on narrow N once ran as a forced K split and a second launch that added the
 // partials; the plan is now free, and a split ends inside its launch (us per call, weights
 // cold, one box: 4096x4096 at M = 33 / 64 8.6 / 8.5 -> 6.8 / 6.6, 4096x6144 at 64 10.8 ->
@@ -1003,13 +1003,7 @@ void describe(int M, int N, int K, int sms, bool noalloc, int out[5]) {
   const int kernel = kernel_for(M, N, K, sms, noalloc);
   out[0] = kernel;
   if (kernel == KERNEL_MID) {
-    // reported with the family of its batch: the large-M kernels from their threshold on
-    // (above 192 rows where they take the shape, else the multi-block one), the LDS-DMA
-    // decode kernels below
     const MidShape d = mid_plan(M, N, K, sms, noalloc);
-    out[0] = M > kMidMaxM && !prefill_fits(M, N, K, VAL4, META4) ? KERNEL_GENERAL
-             : M >= prefill_min_m(N, K)                         ? KERNEL_PREFILL
-                                                                : KERNEL_DECODE_DMA;
     out[1] = N / (16 * d.ncb) * ((M + 16 * d.rb - 1) / (16 * d.rb)) * d.splits;
     out[2] = 512;
     out[3] = d.splits;

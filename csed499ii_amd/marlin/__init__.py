@@ -237,15 +237,16 @@ def mul(A, B, C, s, workspace, thread_k=-1, thread_n=-1, sms=-1, max_par=16):
     raise RuntimeError(_lib.last_error() or f"marlin_hip error {err}")
 
 
-_KERNELS = {-1: None, 0: "decode", 1: "large_m", 2: "general", 3: "decode_dma"}
+_KERNELS = {-1: None, 0: "decode", 1: "large_m", 2: "general", 3: "decode_dma", 4: "mid"}
 
 
 def plan_2_4(M: int, K: int, N: int, groupsize: int = 128, thread_k: int = -1, thread_m: int = -1, sms: int = -1,
              noalloc: bool = False) -> dict:
     """The launch plan of a ``mul_2_4`` call on ``A [M, K]`` and an ``N``-column weight
     (``noalloc=True``: of ``mul_2_4_noalloc``), computed on the host without a GPU
-    (``marlin_hip_plan``): kernel, workgroups and K splits of the first launch,
-    threads per workgroup and launches.  ``splits > 1`` means the call uses its
+    (``marlin_hip_plan``): kernel ("decode", "decode_dma", "mid", "large_m", "general";
+    None for an empty problem), workgroups and K splits of the first launch, threads per
+    workgroup and launches.  ``splits > 1`` means the call uses its
     stream's split-K scratch.  Raises like ``mul_2_4`` for shapes it refuses."""
     out = (ctypes.c_int * 5)()
     g = groupsize // 2 if groupsize != -1 else -1

@@ -99,16 +99,16 @@ def test_plan_without_gpu(built_lib):
     assert p["splits"] == 2 and p["workgroups"] == 256 + 2 * 88
     p = marlin.plan_2_4(24, 4096, 22016, sms=256)  # wide N above 16 rows: the 88 tail tiles split in two
     assert p["kernel"] == "decode_dma" and p["splits"] == 2 and p["workgroups"] == 256 + 2 * 88
-    # 1-8 padded rows run the register-ring decode kernel, 16 and 32 the LDS-DMA one
-    # (7B o at 8 rows takes the 8-row batch; 7B qkv at 8 rows the 16-row batch)
-    assert [marlin.plan_2_4(M, 4096, 4096)["kernel"] for M in (1, 4, 8, 9, 16, 32)] == \
-        ["decode"] * 3 + ["decode_dma"] * 3
+    # 1-8 padded rows run the register-ring decode kernel, 16 the LDS-DMA one (7B o at 8
+    # rows takes the 8-row batch; 7B qkv at 8 rows the 16-row batch), more the mid-batch one
+    assert [marlin.plan_2_4(M, 4096, 4096)["kernel"] for M in (1, 4, 8, 9, 16, 17, 32)] == \
+        ["decode"] * 3 + ["decode_dma"] * 2 + ["mid"] * 2
     assert marlin.plan_2_4(8, 4096, 12288)["kernel"] == "decode_dma"
     assert marlin.plan_2_4(24, 4096, 22016, noalloc=True)["splits"] == 1
     assert marlin.plan_2_4(4, 8192, 8192)["splits"] == 1  # 16-column tiles fill the CUs
     assert marlin.plan_2_4(4, 8192, 10240)["splits"] == 4  # long K, wider N: the tail tiles split four ways
-    p = marlin.plan_2_4(64, 4096, 4096)  # below the large-M threshold: one launch
-    assert p["kernel"] == "decode_dma" and p["launches"] == 1
+    p = marlin.plan_2_4(64, 4096, 4096)  # one round of mid-batch tiles: one launch
+    assert p["kernel"] == "mid" and p["launches"] == 1
     for M in (512, 4096):
         p = marlin.plan_2_4(M, 8192, 57344)
         assert p["kernel"] == "large_m" and p["threads"] == 512
@@ -120,7 +120,8 @@ def test_plan_without_gpu(built_lib):
     assert p["splits"] == 2 and p["workgroups"] == 2 * 8192 // 512 * (512 // 64)
     assert marlin.plan_2_4(512, 28672, 8192, sms=256)["splits"] == 4  # long K: 128-row tiles split four ways
     assert marlin.plan_2_4(512, 8192, 8192, noalloc=True)["splits"] == 1
-    assert marlin.plan_2_4(300, 4096, 768)["kernel"] == "general"  # N % 512 != 0
+    assert marlin.plan_2_4(300, 4096, 768)["kernel"] == "mid"  # narrow N, up to 1024 rows
+    assert marlin.plan_2_4(1100, 4096, 768)["kernel"] == "general"  # N % 512 != 0 below 1024 columns
     with pytest.raises(RuntimeError, match="not compatible"):
         marlin.plan_2_4(16, 1000, 512)
 

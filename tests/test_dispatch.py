@@ -1,7 +1,7 @@
 """Which kernels the calls run and with which K splits, on the CPU (tests/launches.py)."""
 import pytest
 
-from csed499ii_amd import _lib
+from csed499ii_amd import marlin
 from tests.launches import build_fake, launches
 
 COUNTERS = 64 * 1024 // 4  # arrival counters of a stream's split-K scratch
@@ -94,3 +94,27 @@ def test_dense_splits_switch(fake, splits):
             assert x["splits"] in (min(splits, K // 256), 1)
             assert x["splits"] == 1 or x["grid"] // x["splits"] <= COUNTERS, (M, K, N, x)
             assert x["splits"] > 1 or splits == 1 or K == 256 or N > 1 << 20, (M, K, N, x)
+
+
+#: kernels of the plan query, by the name of the kernel that runs
+KERNELS = {"sm24_decode_kernel": "decode", "sm24_decode_dma_kernel": "decode_dma", "sm24_mid_kernel": "mid",
+           "sm24_prefill_kernel": "large_m", "sm24_gemm_kernel": "general"}
+
+
+@pytest.mark.parametrize("op", ["2_4", "noalloc"])
+@pytest.mark.parametrize("K,N", [(4096, 4096), (4096, 22016), (8192, 57344), (28672, 8192), (4096, 768), (192, 4096),
+                                 (8192, 1024), (28672, 1024), (1024, 12288)])
+def test_plan_names_what_runs(fake, op, K, N):
+    """The plan query against the launches themselves: kernel, workgroups, threads and
+    launches of calls of 1 to 4096 rows."""
+    g = -1 if K % 128 else 128
+    calls = [[op, M, K, N, g, 256] for M in (1, 4, 8, 16, 17, 24, 32, 33, 64, 65, 96, 97, 131, 192, 193, 300, 640,
+                                             1024, 1025, 4096) if M > 16 or K % 128 == 0]
+    ls = launches(fake, [calls])
+    for _, M, *_ in calls:
+        p = marlin.plan_2_4(M, K, N, g, sms=256, noalloc=op == "noalloc")
+        mine, ls = ls[:p["launches"]], ls[p["launches"]:]
+        assert KERNELS[mine[0]["kernel"]] == p["kernel"], (M, p, mine)
+        assert len(mine) == 1 or {KERNELS[x["kernel"]] for x in mine} <= {"decode", "decode_dma"}, (M, mine)
+        assert (mine[0]["grid"], mine[0]["block"]) == (p["workgroups"], p["threads"]), (M, p, mine)
+    assert not ls

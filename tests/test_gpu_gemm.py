@@ -207,8 +207,7 @@ def test_mid_batches(M, N, K, g):
     odd counts of them (K = 832, 2176), ragged rows, unsplit and split along K;
     column slices against the oracle, nothing past C's end, repeated calls bit-identical."""
     p = marlin.plan_2_4(M, K, N, g)
-    assert p["threads"] == 512 and p["kernel"] in ("decode_dma", "large_m")
-    assert p["launches"] == 1
+    assert p["kernel"] == "mid" and p["launches"] == 1
     wt, A = _problem(M, N, K, g, 8100 + M + K + N)
     buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
     C = buf[:M * N].view(M, N)
@@ -233,7 +232,7 @@ def test_mid_batches_from_17_rows(M, N, K, g):
     agrees, repeated calls bit-identical.  16 rows and wider N stay on the decode kernels."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     p = marlin.plan_2_4(M, K, N, g, sms=cus)
-    assert p["threads"] == 512 and p["kernel"] == "decode_dma" and p["launches"] == 1
+    assert p["kernel"] == "mid" and p["launches"] == 1
     wt, A = _problem(M, N, K, g, 8300 + M + K + N)
     buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
     C, U = buf[:M * N].view(M, N), torch.empty((M, N), dtype=torch.half, device=DEV)
@@ -259,8 +258,7 @@ def test_mid_batches_narrow_n(M, N, K, g):
     none, one k-pair, widths of no other kernel but the multi-block one (768, 256); column
     slices against the oracle, nothing past C's end, repeated calls bit-identical."""
     p = marlin.plan_2_4(M, K, N, g)
-    assert p["threads"] == 512 and p["launches"] == 1
-    assert p["kernel"] == ("general" if N in (256, 768) or K == 64 else "large_m")
+    assert p["kernel"] == "mid" and p["launches"] == 1
     wt, A = _problem(M, N, K, g, 8500 + M + K + N)
     buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
     C = buf[:M * N].view(M, N)
@@ -344,12 +342,12 @@ def test_prefill_two_group_tiles(M, N, K, g):
         assert torch.equal(_run(wt, A), C), "repeated calls differ"
 
 
-@pytest.mark.parametrize("M,N,K,g", [(97, 1280, 256, 128), (200, 1280, 128, -1), (257, 1792, 8192, 128),
-                                     (65, 4352, 1024, -1), (1100, 2816, 640, 128), (640, 9984, 256, 128)])
+@pytest.mark.parametrize("M,N,K,g", [(300, 4352, 128, -1), (200, 4352, 11008, 128), (257, 4864, 4096, -1),
+                                     (1100, 1792, 8192, 128), (1100, 2816, 640, 128), (640, 9984, 256, 128)])
 def test_prefill_ragged_columns(M, N, K, g):
     """Large-M kernel on N a multiple of 256 but not of its 512-column tile: the last
     tile's upper four waves repeat the last chunk and store nothing (64- and 128-row
-    tiles, narrow tiles, unsplit and split along K); every column against the oracle,
+    tiles, unsplit and split along K); every column against the oracle,
     nothing past C's end, and repeated calls bit-identical."""
     assert marlin.plan_2_4(M, K, N, g)["kernel"] == "large_m"
     wt, A = _problem(M, N, K, g, 5300 + M + N)
@@ -374,15 +372,15 @@ def test_prefill_shape_slices(M):
         assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"prefill M={M} slice {c0}")
 
 
-@pytest.mark.parametrize("M,K,N", [(17, 8192, 57344), (33, 4096, 22016), (33, 8192, 10240), (65, 4096, 4096)])
+@pytest.mark.parametrize("M,K,N", [(17, 8192, 57344), (65, 4096, 22016), (65, 28672, 8192), (129, 4096, 12288),
+                                   (193, 4096, 4096)])
 def test_prefill_from_few_rows(M, K, N):
-    """The large-M kernel at the smallest batches routed to it (from 17 rows for the
-    widest N at long K, from 33 for the widest N and for long K at N >= 10240, from 65
-    at N >= 4096): one ragged 64-row
-    tile per 512 columns; first, middle and last column slices against the oracle,
-    and a repeated call is bit-identical."""
+    """The large-M kernel at the smallest batches routed to it (from 17 rows for the widest
+    N at long K; else where the decode and mid-batch kernels end): two-group tiles up to
+    192 rows, narrow tiles in three K splits at 193; first, middle and last column slices
+    against the oracle, and a repeated call is bit-identical."""
     assert marlin.plan_2_4(M, K, N)["kernel"] == "large_m"
-    assert marlin.plan_2_4(M - 1, K, N)["kernel"] in ("decode", "decode_dma")
+    assert marlin.plan_2_4(M - 1, K, N)["kernel"] == ("decode_dma" if M == 17 else "mid")
     wt, A = _problem(M, N, K, 128, 4100 + M)
     C = _run(wt, A)
     assert torch.isfinite(C).all()
