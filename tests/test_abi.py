@@ -281,11 +281,11 @@ def _kernarg_preload(lib_path):
 def test_decode_kernels_preload_their_leading_arguments(built_lib):
     """The decode-sized kernels take the fields their prologue needs first as leading
     scalar arguments, built to be preloaded into SGPRs: the register-ring, LDS-DMA
-    and lane-native decode kernels 14 dwords, the dense Marlin kernel 12; kernels whose
-    first argument is a struct preload nothing."""
+    and lane-native decode kernels and the mid-batch ones 14 dwords, the dense multi-block
+    kernel 12; kernels whose first argument is a struct preload nothing."""
     pre = _kernarg_preload(_lib.LIB_PATH)
     fam = {"sm24_decode_kernel": 14, "sm24_decode_dma_kernel": 14, "sm24_native_decode_kernel": 14,
-           "marlin_dense_kernel": 12, "sm24_prefill_kernel": 0}
+           "sm24_mid_kernel": 14, "marlin_dense_mid_kernel": 14, "marlin_dense_kernel": 12, "sm24_prefill_kernel": 0}
     for part, want in fam.items():
         got = {k: v for k, v in pre.items() if part + "I" in k}
         assert got, part

@@ -171,22 +171,28 @@ def test_decode_llama70b_full_size_slices(K, N, M):
                                      (384, 1536, 512, 128), (640, 2048, 1024, 128),
                                      (80, 16384, 512, 128), (100, 8192, 512, -1), (160, 4096, 512, 128)])
 def test_prefill_kernel_shapes(M, N, K, g):
-    """The large-M kernel: ragged row tiles, 1-3 k-steps, per-column and grouped
-    scales, several column tiles (every XCD ordering branch).  Problems this small
-    have few tiles, so the planner gives them 64-row tiles."""
+    """Small problems of 80-640 rows: ragged row tiles, short K, per-column and grouped
+    scales, every column.  They run the mid-batch kernel; the large-M kernel's own are
+    test_prefill_beyond_mid's."""
+    assert marlin.plan_2_4(M, K, N, g)["kernel"] == "mid"
     wt, A = _problem(M, N, K, g, 900 + M + K)
     C = _run(wt, A)
     _check(wt, A, C, f"prefill M={M} N={N} K={K} g={g}")
     assert torch.equal(_run(wt, A), C), "repeated calls differ"
 
 
-@pytest.mark.parametrize("M,N,K,g", [(300, 512, 8192, -1), (1000, 2048, 8192, 128), (256, 1024, 4096, 128),
-                                     (100, 4096, 4096, 128), (130, 4096, 11008, -1)])
-def test_prefill_split_k(M, N, K, g):
-    """Large-M kernel split along K (few tiles, long K: the planner picks 3-8 splits
-    of 64-row tiles):
-    partials handed off through the scratch, reduced by the last split in split order,
-    so repeated calls agree bit for bit and the counters return to zero."""
+@pytest.mark.parametrize("M,N,K,g,kernel", [
+    (300, 512, 8192, -1, "mid"), (1000, 2048, 8192, 128, "mid"), (256, 1024, 4096, 128, "mid"),
+    (100, 4096, 4096, 128, "mid"), (130, 4096, 11008, -1, "mid"),
+    (256, 4096, 4096, 128, "large_m"), (1030, 512, 8192, -1, "large_m"), (340, 1024, 17408, 128, "large_m"),
+    (1100, 1024, 4096, 128, "large_m"), (129, 2048, 20480, -1, "large_m")])
+def test_prefill_split_k(M, N, K, g, kernel):
+    """Few tiles and long K.  Large-M kernel: 64- and 128-row, narrow and two-group tiles
+    split along K, partials handed off through the scratch, reduced by the last split in
+    split order, so repeated calls agree bit for bit and the counters return to zero.
+    The mid-batch kernel takes the smaller of these calls, unsplit or split likewise."""
+    p = marlin.plan_2_4(M, K, N, g)
+    assert p["kernel"] == kernel and (kernel == "mid" or p["splits"] > 1)
     wt, A = _problem(M, N, K, g, 1700 + M + K)
     C = _run(wt, A)
     _check(wt, A, C, f"prefill split-K M={M} N={N} K={K} g={g}")
@@ -359,6 +365,47 @@ def test_prefill_ragged_columns(M, N, K, g):
     _check(wt, A, C, f"ragged M={M} N={N} K={K} g={g}")
     assert bool((buf[M * N:] == 7.0).all()), "wrote past C"
     assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
+@pytest.mark.parametrize("M,N,K,g", [(1100, 768, 4096, 128), (700, 256, 11008, 128), (1100, 768, 192, -1),
+                                     (300, 4096, 192, -1), (193, 12288, 64, -1), (200, 8192, 4160, -1),
+                                     (1025, 256, 320, -1), (340, 768, 28672, 128)])
+def test_general_kernel(M, N, K, g):
+    """The multi-block kernel, which takes what no other one does: K of an odd number of
+    64-deep steps or narrow N above the mid-batch kernel's rows; split along K and not, one
+    k-step, ragged row tiles; column slices against the oracle, nothing past C's end,
+    repeated calls bit-identical."""
+    assert marlin.plan_2_4(M, K, N, g)["kernel"] == "general"
+    wt, A = _problem(M, N, K, g, 6600 + M + K)
+    buf = torch.full((M * N + 1024,), 7.0, dtype=torch.half, device=DEV)
+    C = buf[:M * N].view(M, N)
+    ws = torch.zeros(N // 128 * 16, dtype=torch.int32, device=DEV)
+    marlin.mul_2_4(A, wt["B"], wt["meta"], C, wt["s"], ws)
+    torch.cuda.synchronize()
+    assert torch.isfinite(C).all() and bool((buf[M * N:] == 7.0).all())
+    t = to_cpu(wt)
+    for c0 in sorted({0, N // 64 - 4}):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"general M={M} {K}x{N} g={g} slice {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(wt, A), C), "repeated calls differ"
+
+
+@pytest.mark.parametrize("M,N,K,g", [(65, 256, 17408, 128), (80, 1024, 28672, 128), (96, 512, 20480, -1)])
+def test_chunked_decode_launches(M, N, K, g):
+    """65-96 rows at long K and narrow N run as decode launches of 32 rows, the last one of
+    1, 16 or 32: column slices against the oracle, repeated calls bit-identical."""
+    p = marlin.plan_2_4(M, K, N, g)
+    assert p["kernel"] == "decode_dma" and p["launches"] == 3
+    wt, A = _problem(M, N, K, g, 6700 + M + K)
+    C = _run(wt, A)
+    assert torch.isfinite(C).all()
+    t = to_cpu(wt)
+    for c0 in sorted({0, N // 64 - 4}):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"chunks M={M} {K}x{N} g={g} slice {c0}")
+    for _ in range(2):
+        assert torch.equal(_run(wt, A), C), "repeated calls differ"
 
 
 @pytest.mark.parametrize("M", [512])

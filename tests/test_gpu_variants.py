@@ -132,6 +132,27 @@ def test_w3_gemm_bit_exact_against_4bit_path(M, K, N):
     assert torch.equal(C3, C4)
 
 
+@pytest.mark.parametrize("M,K,N,kernel", [(1100, 4096, 768, "general"), (700, 11008, 256, "general"),
+                                          (80, 28672, 1024, "decode_dma"), (65, 17408, 256, "decode_dma")])
+def test_rare_kernels_3bit(M, K, N, kernel):
+    """3-bit values and 3-bit metadata on the multi-block kernel (split along K) and on
+    decode launches in a row: bit-identical to the 4-bit calls, which the oracle checks."""
+    assert marlin.plan_2_4(M, K, N)["kernel"] == kernel
+    wt = synth.make_weight(K, N, 51 + M, 128, bits=3, device=DEV)
+    A = synth.make_activation(M, K, 53 + M, device=DEV)
+    B4 = _w3_as_w4(wt["B"])
+    C3, C4, Cm = (torch.full((M, N), float("nan"), dtype=torch.half, device=DEV) for _ in range(3))
+    marlin.mul_2_4_w3(A, wt["B"], wt["meta"], C3, wt["s"], _ws(N))
+    marlin.mul_2_4(A, B4, wt["meta"], C4, wt["s"], _ws(N))
+    marlin.mul_2_4_meta3(A, B4, marlin.pack_meta3(wt["meta"].reshape(-1)), Cm, wt["s"], _ws(N))
+    torch.cuda.synchronize()
+    assert torch.equal(C3, C4) and torch.equal(Cm, C4)
+    t = to_cpu(wt)
+    for c0 in sorted({0, N // 64 - 4}):
+        ref = oracle_gemm(A.cpu().numpy(), slice_cols(t, c0, 4))
+        assert_close(C3[:, 64 * c0:64 * (c0 + 4)].cpu().numpy(), ref, f"3-bit {kernel} M={M} {K}x{N} slice {c0}")
+
+
 MID_CASES = [(64, 4096, 22016), (48, 4096, 4096), (131, 4096, 4096), (96, 2048, 10240), (80, 1024, 12288),
              (40, 8192, 10240), (24, 8192, 8192), (513, 2048, 2048), (300, 4096, 768)]
 
