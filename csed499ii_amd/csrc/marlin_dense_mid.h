@@ -7,9 +7,11 @@
 // as v_mfma_f32_16x16x32_f16 accumulators, and the 8 sums are added in LDS at the end, in
 // wave order.  No barrier runs in the main loop.
 //
-// What bounds it: at few rows the codes (K N / 2 bytes from HBM), above them the
-// activation rows (L2 hits: 128 bytes per row and k-step against 33 per column) on the
-// 64-byte-per-clock path into the compute unit, and the latency of both.  All operands
+// What bounds it: the latency of the one stage that a wave has in flight.  At 4 rows of the
+// 7B shapes (the codes, K N / 2 bytes from HBM) the waves wait half of their life, over 700
+// clocks a read; at 200 rows (the activation rows, 128 bytes per row and k-step against 34
+// per column) 28-30 %, with the matrix cores busy 34-43 % and the path from L2 into a compute
+// unit at 17-29 of its 64 bytes per clock (counters over the life of a wave).  All operands
 // come by LDS-DMA (codes 1 KiB to an instruction, activation rows in whole 128-byte
 // lines) into one stage buffer per wave, refilled as soon as the stage is in registers
 // (buffers for more stages were no faster: see sm24_mid.h).  The kernel this replaces

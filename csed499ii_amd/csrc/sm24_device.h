@@ -204,8 +204,8 @@ struct SpanStamps {
   }
 };
 
-// Large-M kernel (sm24_prefill.hip): output columns per workgroup tile (N must be a
-// multiple) and its launcher.
+// Large-M kernel (sm24_prefill.hip): output columns per workgroup tile (N is a multiple of
+// half of it: the last tile may be half empty) and its launcher.
 constexpr int kDecodeMaxM = 32;       // largest batch of one decode launch (two 16-row blocks)
 constexpr int kDecodeChunkMaxM = 96;  // largest batch run as several decode launches
 constexpr int kPreTileCols = 512;

@@ -663,7 +663,10 @@ int env_choice(const char* name, std::initializer_list<int> allowed, int fallbac
 // four ways (down at M = 1 two ways: 20.3 -> 19.4 us); Llama-2-70B o (N/16 = 2 per
 // CU) keeps 32-column tiles unsplit up to M = 8 (8.55 -> 7.47 us at M = 1).  The 7B
 // sweep (M in {1, 2, 4, 8, 16}) is within noise of the best forced choice per call.
-// MARLIN_HIP_DECODE_TC / _WAVES / _SPLITS / _DEEP override.
+// MARLIN_HIP_DECODE_TC / _WAVES / _SPLITS / _DEEP override.  From 17 rows on only the calls
+// come here that the mid-batch and large-M kernels leave (N above 64 columns per CU at K
+// below 8192 or at widths that the large-M kernel does not take; launches of a batch of
+// 65-96 rows at K above 16384), and with MARLIN_HIP_MID=0 all below the large-M threshold.
 
 bool decode_deep(int K, int splits);
 
@@ -890,11 +893,11 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
          (long long)M * K < (1LL << 31) - 2048 && (long long)K * N < (1LL << 34);
 }
 
-// Tile and K splits of the mid-batch kernel (17-192 rows; narrow N up to 1024), from a cost model fitted to
-// 3000 forced plans (every tile x splits 1-8 on sixteen K x N, 1024x1024 to 8192x57344, M
-// from 12 to 1024, one box; mean error 6 %, the model's choices 1.4 % from the best of
-// each call): a fixed cost, the stages of a wave at the tile's measured stage time, the
-// reduction in LDS (by tile size), and for a split the exchange of the fp32 partials.
+// Tile and K splits of the mid-batch kernel (17-192 rows; narrow N up to 1024), from a cost
+// model fitted to 3000 forced plans (every tile x splits 1-8 on sixteen K x N, 1024x1024 to
+// 8192x57344, M from 12 to 1024, one box; mean error 6 %, the model's choices 1.4 % from the
+// best of each call): a fixed cost, the stages of a wave at the tile's measured stage time,
+// the reduction in LDS (by tile size), and for a split the exchange of the fp32 partials.
 // Only plans of one workgroup per CU in one round are considered (splits == 0: none): a
 // second round loses to the large-M kernel (7B gate_up at M = 96 28.1 against 23.7 us,
 // 4096x12288 at M = 192 26.9 against 22.7), as does K above 16384 beyond 64 rows

@@ -1,4 +1,4 @@
-// Mid-sized batches (17 to 192 rows) of the 2:4 INT4 x FP16 GEMM for gfx950, where one
+// Mid-sized batches (17 to 192 rows, narrow N up to 1024) of the 2:4 INT4 x FP16 GEMM for gfx950, where one
 // workgroup per tile and K split covers the call in one round over the compute units.
 //
 // Work decomposition: a workgroup of 8 waves owns a tile of 16 NCB output columns (64 or
@@ -8,18 +8,20 @@
 // in wave order.  Nothing is shared before that, so no barrier runs in the main loop and
 // the waves of a SIMD fall out of step: one reads LDS or waits while the other computes.
 //
-// What bounds it.  The activation rows, not the weight, are most of a tile's traffic:
-// 128 bytes per row and k-pair against 26 bytes per column.  They are L2 hits, and the
-// path from L2 into a compute unit moves 64 bytes per clock.  So they come by LDS-DMA in
-// whole 128-byte lines, 8 rows to an instruction (every CU reading the same 64 rows of
-// K = 4096: 5.8 us with the launch, against 7.2 in 64-byte pieces and 17 by loads into
-// registers in operand order).  A wave has one stage buffer: it reads the due stage into
-// registers in one go, sends for the next one into the same buffer and computes meanwhile.
-// More stages in flight were slower on every call (buffers for 1 / 2 / 4 stages, us: 7B
-// qkv at M = 64 12.3 / 13.8 / 13.8, o at M = 131 8.6 / 9.6 / 9.8, 70B o at M = 64 15.3 /
-// 15.9 / 16.8): a wave's DMAs return in order, so the first stage waits for less, and the
-// smaller LDS lets two workgroups share a compute unit.  4, 12 and 16 waves were slower
-// than 8.
+// What bounds it: the latency of the one stage that a wave has in flight, no unit's rate.
+// On 7B qkv and o at 64 and 131 rows the waves wait 43-48 % of their life; the matrix cores
+// are busy 9-18 % of it, LDS 29-40 %, and the path from L2 into a compute unit carries 20-28
+// of its 64 bytes per clock, at 320-370 clocks per read (counters over the life of a wave).
+// The activation rows are most of that traffic: 128 bytes per row and k-pair against 26 per
+// column.  So they come by LDS-DMA in whole 128-byte lines, 8 rows to an instruction (every
+// CU reading the same 64 rows of K = 4096: 5.8 us with the launch, against 7.2 in 64-byte
+// pieces and 17 by loads into registers in operand order).  A wave has one stage buffer: it
+// reads the due stage into registers in one go, sends for the next one into the same buffer
+// and computes meanwhile.  Buffers for more stages were slower on every call (1 / 2 / 4
+// stages, us: 7B qkv at M = 64 12.3 / 13.8 / 13.8, o at M = 131 8.6 / 9.6 / 9.8, 70B o at
+// M = 64 15.3 / 15.9 / 16.8): the LDS they take goes from the tile (four 16-row blocks of
+// one stage are 136 KiB over the 8 waves) or from a second workgroup on the compute unit.
+// 4, 12 and 16 waves were slower than 8.
 //
 // us per call on one box, against the decode launches of up to 32 rows or the large-M
 // kernel: M = 64 7B qkv 18.9 -> 12.4, o 14.6 -> 6.6, gate_up 21.3 -> 19.0,

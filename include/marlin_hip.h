@@ -17,7 +17,7 @@
  *
  * The planner may split K (decode calls at wide N or long K, decode calls whose
  * column tiles leave a tail of at most half the compute units past whole rounds,
- * where only the tail tiles are split, large-M calls with few column tiles,
+ * where only the tail tiles are split, mid-batch and large-M calls with few tiles,
  * lane-native calls at 5-16 rows whose tiles cover too few compute units, and at
  * 2-4 rows when K >= 16384).  The split-K scratch (fp32 partials and
  * arrival counters) is uncached device memory that the library allocates per
@@ -28,6 +28,9 @@
  * reference keeps its split-K locks there, common/mem.h:111-142).
  * The counters are zeroed at allocation and each is returned to zero by the last
  * workgroup that arrives on it, so no buffer needs to be zeroed by the caller.
+ * Host threads may issue calls on one stream at the same time: a call hands its
+ * partials over inside one launch, and an expansion into the stream's staging buffer
+ * and the kernel that reads it reach the stream together.
  * During stream capture nothing can be allocated: a call whose stream has no large
  * enough scratch yet then runs without splitting K (same result within the GEMM
  * tolerance, a different summation order), and one that needs a larger staging

@@ -159,8 +159,9 @@ MID_CASES = [(64, 4096, 22016), (48, 4096, 4096), (131, 4096, 4096), (96, 2048, 
 
 @pytest.mark.parametrize("M,K,N", MID_CASES)
 def test_mid_batches_3bit(M, K, N):
-    """The mid-batch kernel (17-192 rows, narrow N up to 1024) on 3-bit metadata and 3-bit values: the same
-    tiles and order of sums as 4-bit operands, so bit-identical to the 4-bit calls."""
+    """The mid-batch kernel (17-192 rows, narrow N up to 1024) on 3-bit metadata and 3-bit
+    values: the same tiles and order of sums as 4-bit operands, so bit-identical to the
+    4-bit calls."""
     assert marlin.plan_2_4(M, K, N)["kernel"] == "mid"
     A = synth.make_activation(M, K, 7 + M, device=DEV)
 
