@@ -914,7 +914,9 @@ bool prefill_fits(int M, int N, int K, int vf, int mf) {
 // 33-64 rows on narrow N once ran as a forced K split and a second launch that added the
 // partials; the plan is now free, and a split ends inside its launch (us per call, weights
 // cold, one box: 4096x4096 at M = 33 / 64 8.6 / 8.5 -> 6.8 / 6.6, 4096x6144 at 64 10.8 ->
-// 7.5, 8192x7936 17.7 -> 15.5, 11008x4096 14.2 -> 12.9, 28672x4096 25.3 -> 25.4).
+// 7.5, 8192x7936 17.7 -> 15.5, 11008x4096 14.2 -> 12.9, 28672x4096 25.3 -> 25.4; at K from
+// 16384 with five and more splits up to 6 % slower, 16384x6144 at 62 21.5 -> 22.8: the last
+// workgroup of a tile adds alone what that launch spread over the chip).
 // MARLIN_HIP_MID=0 turns the kernel off (read once).
 constexpr int kMidMinM = 17, kMidMaxM = 192;
 // Narrow N (below 4096) leaves the large-M kernel a few workgroups that split K up to eight
